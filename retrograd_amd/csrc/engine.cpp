@@ -494,6 +494,7 @@ void Engine::build_buffers() {
         moe_off_.alloc((size_t)(NE + 1) * 4);
         moe_tok_.alloc(slots * 4);
         moe_pair_.alloc(slots * 4);
+        moe_items_.alloc(rk::moe_items(B, KU, NE) * sizeof(int2));
         moe_q_.alloc((size_t)B * KU * 4);
         moe_h_.alloc(rk::act_halves((int)slots, FE) * 2);
         hip_check(hipMemsetAsync(moe_h_.ptr, 0, moe_h_.bytes, stream_), "hipMemsetAsync");
@@ -1668,6 +1669,7 @@ void Engine::forward(int T, int n_out, int n_tiles, int n_items, bool one_token_
             mb.mx_ops = moe_mx_ops_.as<uint8_t>(); mb.mx_scales = moe_mx_scales_.as<uint8_t>(); mb.mx_h = moe_mx_h_.as<float>();
             mb.mx_slots = moe_mx_slots_;
             mb.pair_of_q = moe_pair_.as<int32_t>();
+            mb.items = moe_items_.as<int2>();
             pending = rk::moe_ffn(stream_, ml, ms, act_e, T, x, mb, true);     // the next norm adds the experts' weighted sum
             prof_end(PC_GATEUP, pt_);
             continue;

@@ -279,7 +279,9 @@ struct MoeBuffers {            // device scratch of one step, sized with moe_slo
     size_t mx_slots = 0;
     int32_t * pair_of_q = nullptr;   // [slots] the pair (token * k_used + choice) of a slot, -1 for padding; or null: then the
                                      // down projection leaves its rows in slot order instead of pair order
+    int2 * items = nullptr;          // [moe_items] their number, then (expert, first pair) of every work item of the grouped products
 };
+size_t moe_items(int n_tokens, int k_used, int n_expert);
 size_t moe_slots(int n_tokens, int k_used, int n_expert);
 // x[t] += sum over the token's k_used experts of w * down_e(silu(gate_e xn) * (up_e xn))
 // With defer_combine the weighted sum is not added to x: it is returned as gathered slices for the next rmsnorm_act.

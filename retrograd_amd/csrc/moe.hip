@@ -27,6 +27,8 @@
 // half scale multiplies): four instructions decode a lane's eight weights.
 #include "dev_common.hpp"
 
+#include <type_traits>
+
 namespace rk {
 
 bool moe_can_pack(int type, int64_t K, int64_t N) {
@@ -106,6 +108,11 @@ template <> struct Tile<WT_MXFP4> {
         q0 = *(const u4 *)(tile + 128 + lane * 16);
         q1 = *(const u4 *)(tile + 128 + 1024 + lane * 16);
     }
+    // what k-steps 4 H .. 4 H + 3 need
+    template <int H> __device__ __forceinline__ void load_half(const uint8_t * tile, int lane) {
+        hdr = *(const uint2 *)(tile + (uint32_t)((lane & 15) * 8));
+        (H ? q1 : q0) = *(const u4 *)(tile + 128 + H * 1024 + (uint32_t)(lane * 16));
+    }
     // half of 2^(x - 127): the E8M0 scale of doubled magnitudes
     __device__ __forceinline__ float scale(int s) const {
         const uint32_t x = ((s < 4 ? hdr.x : hdr.y) >> (8 * (s & 3))) & 0xff;
@@ -131,6 +138,11 @@ template <> struct Tile<WT_Q8_0> {
         hdr = *(const u4 *)(tile + (lane & 15) * 16);
 #pragma unroll
         for (int j = 0; j < 4; ++j) q[j] = *(const u4 *)(tile + 256 + j * 1024 + lane * 16);
+    }
+    template <int H> __device__ __forceinline__ void load_half(const uint8_t * tile, int lane) {
+        hdr = *(const u4 *)(tile + (uint32_t)((lane & 15) * 16));
+        q[2 * H] = *(const u4 *)(tile + 256 + 2 * H * 1024 + (uint32_t)(lane * 16));
+        q[2 * H + 1] = *(const u4 *)(tile + 256 + (2 * H + 1) * 1024 + (uint32_t)(lane * 16));
     }
     __device__ __forceinline__ float scale(int s) const {
         const uint32_t sw = hdr[s >> 1];
@@ -180,6 +192,11 @@ template <bool FIVE> struct TileQ45 {
         q1 = *(const u4 *)(tile + 256 + 1024 + lane * 16);
         top0 = FIVE ? *(const uint32_t *)(tile + 2304 + lane * 4) : 0u;
         top1 = FIVE ? *(const uint32_t *)(tile + 2304 + 256 + lane * 4) : 0u;
+    }
+    template <int H> __device__ __forceinline__ void load_half(const uint8_t * tile, int lane) {
+        hdr = *(const u4 *)(tile + (uint32_t)((lane & 15) * 16));
+        (H ? q1 : q0) = *(const u4 *)(tile + 256 + H * 1024 + (uint32_t)(lane * 16));
+        (H ? top1 : top0) = FIVE ? *(const uint32_t *)(tile + 2304 + H * 256 + (uint32_t)(lane * 4)) : 0u;
     }
     __device__ __forceinline__ Q4KOperand prep(int s) const {
         const Q4KScales s4 = q4k_scales(hdr);
@@ -244,6 +261,13 @@ template <> struct Tile<WT_Q6_K> {
         ql1 = *(const u4 *)(tile + 288 + 1024 + lane * 16);
         qh0 = *(const uint2 *)(tile + 2336 + lane * 8);
         qh1 = *(const uint2 *)(tile + 2336 + 512 + lane * 8);
+    }
+    template <int H> __device__ __forceinline__ void load_half(const uint8_t * tile, int lane) {
+        lane_ = lane;
+        sc = *(const u4 *)(tile + (uint32_t)((lane & 15) * 16));
+        dpair = *(const uint32_t *)(tile + 256 + (uint32_t)(((lane & 15) >> 1) * 4));
+        (H ? ql1 : ql0) = *(const u4 *)(tile + 288 + H * 1024 + (uint32_t)(lane * 16));
+        (H ? qh1 : qh0) = *(const uint2 *)(tile + 2336 + H * 512 + (uint32_t)(lane * 8));
     }
     __device__ __forceinline__ Q6KOperand prep(int s) const {
         const int j = s & 3;
@@ -615,6 +639,231 @@ void k_moe_down(MoeArgs a) {
     }
 }
 
+// ---- many pairs per expert -------------------------------------------------------------------------------------
+//
+// The kernels above multiply a weight tile with 32 pairs per trip through memory and decode, from rows gathered in
+// pieces of 16 bytes; with a hundred pairs per expert (a prompt) they run at a third of the matrix rate. Here a
+// workgroup owns (up to) 64 pairs of an expert and RT row tiles per wave and matrix, so a decoded operand meets four
+// token tiles and a staged token tile RT row tiles per matrix. Same products, same order of additions: the same bits.
+// 1818 tokens over 128 MXFP4 experts of 768 x 2048, 8 per token: gate/up 668 (514 at best) -> 247 us, 0.76 PFLOP/s
+// counting the hi and the lo product, down 234 -> 131 us. Matrix issue bounds it: per k-step and wave 32 matrix
+// instructions beside 64 scale multiply-adds, 28 decode instructions and 8 LDS reads.
+
+// The activation planes as rows for gathering: [token][k / 32][hi, lo][32 halves], so that the pieces of a row that a
+// staging request takes are 64 contiguous bytes (in the operand order they are 16 bytes each, a quarter of a sector).
+__global__ __launch_bounds__(256) void k_moe_rows(const __half * __restrict__ x, int K, int T, __half * __restrict__ rows) {
+    const int lane = threadIdx.x & 63;
+    const size_t unit = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);         // [chunk][k / 32][hl][tile of 16 tokens]
+    const size_t per_chunk = (size_t)(K >> 5) * 8;
+    const int chunk = (int)(unit / per_chunk), rem = (int)(unit % per_chunk);
+    const int tok = chunk * 64 + (rem & 3) * 16 + (lane & 15);
+    const u4 v = *(const u4 *)(x + (size_t)chunk * act_chunk_halves(K) + (size_t)rem * 512 + lane * 8);
+    if (tok < T) *(u4 *)(rows + (size_t)tok * K * 2 + (size_t)(rem >> 2) * 32 + (lane >> 4) * 8) = v;
+}
+
+struct GroupedArgs {
+    const uint8_t * w[2];      // gate and up, or down
+    const __half * x;          // gate_up: rows as k_moe_rows leaves them; down: the hidden planes by slot
+    __half * h;                // gate_up output
+    float * out_pair;          // down output
+    const int2 * items;
+    const int32_t * expert_n, * off_pad, * tok_of_q, * pair_of_q;
+    int K, N, groups;          // groups: workgroups per item
+};
+
+constexpr int kGroupTokens = 64;                   // pairs of a work item
+constexpr int kHalfTile = 4 * 2 * 1024;            // staged bytes of a token tile per 128 columns (4 k-steps, hi and lo)
+constexpr int kHalfBuf = 4 * kHalfTile;            // ... of four token tiles
+constexpr int kGroupPad = 4;                       // floats between the rows of the epilogue's exchange
+
+// Workgroup b runs on XCD b % 8: the items are dealt to the XCDs, and the workgroups of one item, which read the same
+// rows, follow each other on one XCD.
+__device__ __forceinline__ bool grouped_item(const GroupedArgs & a, int2 & item, int & group) {
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int i = (j / a.groups) * 8 + xcd;
+    group = j % a.groups;
+    if (i >= a.items[0].x) return false;
+    const int2 v = a.items[1 + i];
+    item = make_int2(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y));
+    return true;
+}
+
+// acc[m][r][t] += the products of NT token tiles with RT row tiles of MATS matrices over all of K. The unit of the
+// pipeline is half a super-block (128 columns): its weights (registers) and activations (global -> LDS) are requested
+// while the half before it is multiplied. The waits are written here: a half is 128 matrix instructions a wave and
+// more, longer than any request takes, so each half begins with everything requested before it having landed.
+template <int TYPE, int MATS, int RT, int NT>
+__device__ __forceinline__ void grouped_product(const uint8_t * const (&w)[MATS], int nsb, const uint8_t * x, uint32_t x_lane, int x_step, int x_lo,
+                                                uint8_t * stage, f4 (&acc)[MATS][RT][NT]) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lds0 = lds_offset(stage);
+    const size_t tile_bytes = (size_t)nsb * Tile<TYPE>::BYTES;
+    auto request_x = [&](int half) __attribute__((always_inline)) {       // wave t stages token tile t
+        if (wave >= NT) return;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl)
+                lds_dma16(x + (size_t)(half * 4 + s) * x_step + hl * x_lo, x_lane,
+                          lds0 + (uint32_t)(half & 1) * kHalfBuf + (uint32_t)((s * 2 + hl) * 4 + wave) * 1024u);
+    };
+    Tile<TYPE> w0[MATS][RT], w1[MATS][RT];         // of the first and the second half
+    auto multiply = [&](int half, auto first, const Tile<TYPE> (&wt)[MATS][RT]) __attribute__((always_inline)) {
+        const uint8_t * buf = stage + (half & 1) * kHalfBuf;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            decltype(wt[0][0].prep(0)) op[MATS][RT];
+#pragma unroll
+            for (int m = 0; m < MATS; ++m)
+#pragma unroll
+                for (int r = 0; r < RT; ++r) op[m][r] = wt[m][r].prep(decltype(first)::value + s);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const h8 hi = *(const h8 *)(buf + ((s * 2) * 4 + t) * 1024 + lane * 16);
+                const h8 lo = *(const h8 *)(buf + ((s * 2 + 1) * 4 + t) * 1024 + lane * 16);
+#pragma unroll
+                for (int m = 0; m < MATS; ++m)
+#pragma unroll
+                    for (int r = 0; r < RT; ++r) mac(op[m][r], hi, lo, acc[m][r][t]);
+#pragma unroll
+                for (int m = 0; m < MATS; ++m)
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)      // (or the additions sink behind the next requests, and every product is spilled)
+                        asm volatile("" : "+v"(acc[m][r][t]));
+            }
+        }
+    };
+#pragma unroll
+    for (int m = 0; m < MATS; ++m)
+#pragma unroll
+        for (int r = 0; r < RT; ++r) w0[m][r].template load_half<0>(w[m] + r * tile_bytes, lane);
+    request_x(0);
+#pragma unroll 1
+    for (int sb = 0; sb < nsb; ++sb) {
+        const size_t at = (size_t)sb * Tile<TYPE>::BYTES, next = (size_t)min(sb + 1, nsb - 1) * Tile<TYPE>::BYTES;
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();               // buffer 0 holds the first half; none still reads buffer 1
+        request_x(2 * sb + 1);
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) w1[m][r].template load_half<1>(w[m] + r * tile_bytes + at, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(2 * sb, std::integral_constant<int, 0>{}, w0);
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+        if (sb + 1 < nsb) request_x(2 * sb + 2);
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) w0[m][r].template load_half<0>(w[m] + r * tile_bytes + next, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(2 * sb + 1, std::integral_constant<int, 4>{}, w1);
+    }
+}
+
+template <int TYPE, int RT, int NT>
+__device__ __forceinline__ void grouped_gate_up(const GroupedArgs & a, int2 item, int group, int n_e, uint8_t * stage) {
+    constexpr int COLS = 64 * RT, LD = COLS + kGroupPad;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g = lane >> 4, nsb = a.K >> 8;
+    const int qb = __builtin_amdgcn_readfirstlane(a.off_pad[item.x]) + item.y, n = min(n_e - item.y, kGroupTokens);
+    const size_t tile0 = (size_t)item.x * (a.N / 16) + group * (4 * RT) + wave * RT;
+    const uint8_t * const w[2] = {a.w[0] + tile0 * nsb * Tile<TYPE>::BYTES, a.w[1] + tile0 * nsb * Tile<TYPE>::BYTES};
+    // padding pairs read token 0 and are never stored
+    const int at = wave * 16 + r16;
+    const int tok = at < n ? a.tok_of_q[qb + at] : 0;
+    f4 acc[2][RT][NT];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[m][r][t] = (f4){0.f, 0.f, 0.f, 0.f};
+    grouped_product<TYPE, 2, RT, NT>(w, nsb, (const uint8_t *)a.x, (uint32_t)tok * (uint32_t)a.K * 4u + g * 16u, 128, 64, stage, acc);
+    // SwiGLU, and through LDS so that a lane stores eight columns of a pair at once
+    float * ex = (float *)stage;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float gv = acc[0][r][t][i];
+                ex[(t * 16 + 4 * g + i) * LD + (wave * RT + r) * 16 + r16] =
+                    fminf(fmaxf((gv / (1.0f + __expf(-gv))) * acc[1][r][t][i], -65504.0f), 65504.0f);
+            }
+    __syncthreads();
+    for (int j = threadIdx.x; j < n * (COLS / 8); j += 256) {
+        const int row = j / (COLS / 8), c = (j % (COLS / 8)) * 8;
+        h8 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float v = ex[row * LD + c + i];
+            hi[i] = (_Float16)v;
+            lo[i] = (_Float16)(v - (float)hi[i]);
+        }
+        *(h8 *)(a.h + act_at(qb + row, group * COLS + c, 0, a.N)) = hi;
+        *(h8 *)(a.h + act_at(qb + row, group * COLS + c, 1, a.N)) = lo;
+    }
+}
+
+template <int TYPE, int RT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_moe_grouped_gate_up(GroupedArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t stage[2 * kHalfBuf];
+    int2 item;
+    int group;
+    if (!grouped_item(a, item, group)) return;
+    const int n_e = __builtin_amdgcn_readfirstlane(a.expert_n[item.x]), nt = (min(n_e - item.y, kGroupTokens) + 15) / 16;
+    if (nt > 3) grouped_gate_up<TYPE, RT, 4>(a, item, group, n_e, stage);
+    else if (nt == 3) grouped_gate_up<TYPE, RT, 3>(a, item, group, n_e, stage);
+    else if (nt == 2) grouped_gate_up<TYPE, RT, 2>(a, item, group, n_e, stage);
+    else grouped_gate_up<TYPE, RT, 1>(a, item, group, n_e, stage);
+}
+
+template <int TYPE, int RT, int NT>
+__device__ __forceinline__ void grouped_down(const GroupedArgs & a, int2 item, int group, int n_e, uint8_t * stage) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g = lane >> 4, nsb = a.K >> 8;
+    const int qb = __builtin_amdgcn_readfirstlane(a.off_pad[item.x]) + item.y, n = min(n_e - item.y, kGroupTokens);
+    const int tile = group * (4 * RT) + wave * RT;
+    const uint8_t * const w[1] = {a.w[0] + ((size_t)item.x * (a.N / 16) + tile) * nsb * Tile<TYPE>::BYTES};
+    f4 acc[1][RT][NT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[0][r][t] = (f4){0.f, 0.f, 0.f, 0.f};
+    // a tile of 16 slots lies in the planes as the operand wants it: 1 KiB per k-step and half (every row of a tile that
+    // holds a pair lies in the expert's padded slot range)
+    const int slot = qb + min(wave, NT - 1) * 16;
+    const uint8_t * x = (const uint8_t *)(a.x + act_at(slot, 0, 0, a.K));
+    grouped_product<TYPE, 1, RT, NT>(w, nsb, x, (uint32_t)lane * 16u, 8192, 4096, stage, acc);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int at = t * 16 + 4 * g + i;
+            if (at >= n) continue;
+            const int row = a.pair_of_q ? a.pair_of_q[qb + at] : qb + at;
+#pragma unroll
+            for (int r = 0; r < RT; ++r) a.out_pair[(size_t)row * a.N + (tile + r) * 16 + r16] = acc[0][r][t][i];
+        }
+}
+
+template <int TYPE, int RT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_moe_grouped_down(GroupedArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t stage[2 * kHalfBuf];
+    int2 item;
+    int group;
+    if (!grouped_item(a, item, group)) return;
+    const int n_e = __builtin_amdgcn_readfirstlane(a.expert_n[item.x]), nt = (min(n_e - item.y, kGroupTokens) + 15) / 16;
+    if (nt > 3) grouped_down<TYPE, RT, 4>(a, item, group, n_e, stage);
+    else if (nt == 3) grouped_down<TYPE, RT, 3>(a, item, group, n_e, stage);
+    else if (nt == 2) grouped_down<TYPE, RT, 2>(a, item, group, n_e, stage);
+    else grouped_down<TYPE, RT, 1>(a, item, group, n_e, stage);
+}
+
 // Router logits on the f32 matrix instruction (32x32x2: exact f32 products, f32 sums): one wave per (32 experts,
 // 32 tokens, 128 columns of K) leaves its sums as a K-slice [slice][token][expert]; k_moe_route adds the slices
 // in slice order. The rows are the f32 router weights, the tokens' values hi + lo of the activation planes.
@@ -712,75 +961,73 @@ __global__ __launch_bounds__(64) void k_moe_route(const float * __restrict__ log
 }
 
 // Stable counting sort of the pairs by expert, every expert's range padded to a
-// multiple of 16 slots. One workgroup of 1024 threads.
-__global__ __launch_bounds__(1024) void k_moe_group(const int32_t * __restrict__ sel, int n_pairs, int n_expert, int k_used,
-                                                    int32_t * __restrict__ expert_n, int32_t * __restrict__ off_pad,
-                                                    int32_t * __restrict__ tok_of_q, int32_t * __restrict__ q_of_pair,
-                                                    int32_t * __restrict__ pair_of_q) {
-    __shared__ int cnt[256];
-    __shared__ int base[256];
-    __shared__ int wcnt[16][256];
-    __shared__ int total_pad;
-    __shared__ int wsum[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid < 256) cnt[tid] = 0;
-    for (int i = tid; i < 16 * 256; i += 1024) (&wcnt[0][0])[i] = 0;
+// multiple of 16 slots, and the work items of the grouped products: (expert, first pair) per kGroupTokens pairs of
+// an expert, behind their number in items[0].x. One workgroup per expert: each counts all pairs (LDS), which gives it
+// every expert's place, and then places its own - four waves, a contiguous quarter of the pairs each, ranks from
+// ballots - so nothing passes between workgroups. (One workgroup that places 1024 pairs per turn, three barriers and
+// 64 shuffles each, took 67 us for 14544 pairs and 6.8 us for 1024; this takes 16.9 and 5.2.)
+__global__ __launch_bounds__(256) void k_moe_group(const int32_t * __restrict__ sel, int n_pairs, int n_expert, int k_used,
+                                                   int32_t * __restrict__ expert_n, int32_t * __restrict__ off_pad,
+                                                   int32_t * __restrict__ tok_of_q, int32_t * __restrict__ q_of_pair,
+                                                   int32_t * __restrict__ pair_of_q, int2 * __restrict__ items) {
+    __shared__ int cnt[256], slots_to[4], items_to[4], wave_n[4];
+    __shared__ int place, item_place;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, e = blockIdx.x;
+    cnt[tid] = 0;
     __syncthreads();
-    for (int p = tid; p < n_pairs; p += 1024) atomicAdd(&cnt[sel[p]], 1);
+    const int part = ((n_pairs + 255) / 256) * 64;            // a wave's pairs, whole turns of 64
+    const int p_lo = min(wave * part, n_pairs), p_hi = min(p_lo + part, n_pairs);
+    int mine = 0;
+    for (int p0 = p_lo; p0 < p_hi; p0 += 512) {               // eight turns' loads in flight together
+        int v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { const int p = p0 + u * 64 + lane; v[u] = p < p_hi ? sel[p] : -1; }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (v[u] >= 0) atomicAdd(&cnt[v[u]], 1);
+            mine += __popcll(__ballot(v[u] == e));
+        }
+    }
+    if (lane == 0) wave_n[wave] = mine;
     __syncthreads();
-    // exclusive prefix sums of the padded counts: a scan inside each of the first four waves, then the waves' totals
-    int padded = 0, incl = 0;
-    if (tid < 256) {
-        padded = tid < n_expert ? (cnt[tid] + 15) & ~15 : 0;
-        incl = padded;
+    // exclusive prefix sums over the experts of the padded counts and of the items
+    {
+        const int n = tid < n_expert ? cnt[tid] : 0;
+        const int padded = (n + 15) & ~15, it = (n + kGroupTokens - 1) / kGroupTokens;
+        int a = padded, b = it;
         for (int o = 1; o < 64; o <<= 1) {
-            const int up = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += up;
+            const int ua = __shfl_up(a, o, 64), ub = __shfl_up(b, o, 64);
+            if (lane >= o) { a += ua; b += ub; }
         }
-        if (lane == 63) wsum[wave] = incl;
+        if (lane == 63) { slots_to[wave] = a; items_to[wave] = b; }
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) { a += slots_to[w]; b += items_to[w]; }
+        if (tid == e) { place = a - padded; item_place = b - it; }
+        if (e == 0 && tid < n_expert) { expert_n[tid] = n; off_pad[tid] = a - padded; }
+        if (e == 0 && tid == n_expert - 1) { off_pad[n_expert] = a; items[0] = make_int2(b, 0); }
     }
     __syncthreads();
-    if (tid < 256) {
-        int before = 0;
-        for (int w = 0; w < wave; ++w) before += wsum[w];
-        const int at = before + incl - padded;
-        if (tid < n_expert) {
-            off_pad[tid] = at;
-            base[tid] = at;
-            expert_n[tid] = cnt[tid];
+    const int n_e = cnt[e], base = place;
+    for (int i = tid; i * kGroupTokens < n_e; i += 256) items[1 + item_place + i] = make_int2(e, i * kGroupTokens);
+    for (int i = n_e + tid; i < ((n_e + 15) & ~15); i += 256) tok_of_q[base + i] = -1;
+    int at = base;
+    for (int w = 0; w < wave; ++w) at += wave_n[w];
+    for (int p0 = p_lo; p0 < p_hi; p0 += 512) {
+        int v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { const int p = p0 + u * 64 + lane; v[u] = p < p_hi ? sel[p] : -1; }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const uint64_t hits = __ballot(v[u] == e);
+            if (v[u] == e) {
+                const int p = p0 + u * 64 + lane;
+                const int pos = at + __popcll(hits & ((1ull << lane) - 1));
+                q_of_pair[p] = pos;
+                tok_of_q[pos] = p / k_used;
+                if (pair_of_q) pair_of_q[pos] = p;
+            }
+            at += __popcll(hits);
         }
-        if (tid == n_expert - 1) {
-            off_pad[n_expert] = at + padded;
-            total_pad = at + padded;
-        }
-    }
-    __syncthreads();
-    for (int q = tid; q < total_pad; q += 1024) tok_of_q[q] = -1;
-    __syncthreads();
-    for (int c0 = 0; c0 < n_pairs; c0 += 1024) {
-        const int p = c0 + tid;
-        const int e = p < n_pairs ? sel[p] : -1;
-        int rank = 0;
-        for (int i = 0; i < 64; ++i) {
-            const int other = __shfl(e, i, 64);
-            if (other == e && i < lane) ++rank;
-        }
-        if (e >= 0) atomicMax(&wcnt[wave][e], rank + 1);
-        __syncthreads();
-        if (e >= 0) {
-            int pos = base[e] + rank;
-            for (int w = 0; w < wave; ++w) pos += wcnt[w][e];
-            q_of_pair[p] = pos;
-            tok_of_q[pos] = p / k_used;
-            if (pair_of_q) pair_of_q[pos] = p;
-        }
-        __syncthreads();
-        if (tid < n_expert) {
-            int add = 0;
-            for (int w = 0; w < 16; ++w) { add += wcnt[w][tid]; wcnt[w][tid] = 0; }
-            base[tid] += add;
-        }
-        __syncthreads();
     }
 }
 
@@ -798,6 +1045,30 @@ __global__ __launch_bounds__(256) void k_moe_combine(const float * __restrict__ 
     }
     f4 * dst = (f4 *)(x + (size_t)t * E + c);
     *dst += acc;
+}
+
+// Row tiles per wave and matrix of the grouped products: what two waves a SIMD have registers for (half as many: 2 %
+// slower at 16 pairs per expert, 13 to 19 % at 128).
+constexpr int kGroupRtGateUp = 2, kGroupRtDown = 4;
+static unsigned grouped_blocks(int T, const MoeShape & sh, int groups) {
+    const size_t items = (size_t)T * sh.k_used / kGroupTokens + std::min((size_t)sh.n_expert, (size_t)T * sh.k_used);
+    return (unsigned)((items + 7) / 8 * 8 * (size_t)groups);
+}
+template <int TYPE> static void grouped_gate_up_launch(hipStream_t s, GroupedArgs a, int T, const MoeShape & sh) {
+    constexpr int RT = kGroupRtGateUp;
+    a.groups = a.N / (64 * RT);
+    hipLaunchKernelGGL((k_moe_grouped_gate_up<TYPE, RT>), dim3(grouped_blocks(T, sh, a.groups)), dim3(256), 0, s, a);
+    check_launch("moe_grouped_gate_up");
+}
+template <int TYPE> static void grouped_down_launch(hipStream_t s, GroupedArgs a, int T, const MoeShape & sh) {
+    constexpr int RT = kGroupRtDown;
+    a.groups = a.N / (64 * RT);
+    hipLaunchKernelGGL((k_moe_grouped_down<TYPE, RT>), dim3(grouped_blocks(T, sh, a.groups)), dim3(256), 0, s, a);
+    check_launch("moe_grouped_down");
+}
+
+size_t moe_items(int n_tokens, int k_used, int n_expert) {
+    return (size_t)n_tokens * k_used / kGroupTokens + n_expert + 1;
 }
 
 size_t moe_slots(int n_tokens, int k_used, int n_expert) {
@@ -844,8 +1115,8 @@ Slices moe_ffn(hipStream_t s, const MoeLayer & L, const MoeShape & sh, const Act
         hipLaunchKernelGGL(k_moe_route, dim3(T), dim3(64), 0, s, b.logits, 1, (size_t)0, sh.n_expert, sh.k_used, b.sel, b.wgt);
     }
     check_launch("moe_route");
-    hipLaunchKernelGGL(k_moe_group, dim3(1), dim3(1024), 0, s, b.sel, T * sh.k_used, sh.n_expert, sh.k_used, b.expert_n,
-                       b.off_pad, b.tok_of_q, b.q_of_pair, b.pair_of_q);
+    hipLaunchKernelGGL(k_moe_group, dim3(sh.n_expert), dim3(256), 0, s, b.sel, T * sh.k_used, sh.n_expert, sh.k_used, b.expert_n,
+                       b.off_pad, b.tok_of_q, b.q_of_pair, b.pair_of_q, b.items);
     check_launch("moe_group");
     MoeArgs a {};
     a.expert_n = b.expert_n; a.off_pad = b.off_pad; a.tok_of_q = b.tok_of_q; a.n_expert = sh.n_expert;
@@ -866,15 +1137,36 @@ Slices moe_ffn(hipStream_t s, const MoeLayer & L, const MoeShape & sh, const Act
                      b.out_pair);
         return combine(false);
     }
+    // Many pairs per expert: the grouped products, which give the same bits. Us per layer (all launches of the block) on
+    // the 128-expert shape, two-tile kernels / grouped, at 16, 24, 32, 64 and 128 pairs per expert: MXFP4 156 / 153,
+    // 193 / 172, 236 / 203, 429 / 277, 892 / 454; Q4_K + Q6_K 242 / 220, 285 / 252, 346 / 280, 577 / 411, 1128 / 672;
+    // Q8_0, whose codes cost least to decode again, 213 / 220, 248 / 246, 312 / 266, 566 / 357, 1159 / 554.
+    // (Rows are gathered by 32-bit byte offsets.)
+    const size_t many = L.gate.type == WT_Q8_0 ? 24 : 16;
+    const bool grouped = b.items && (size_t)T * sh.k_used >= many * sh.n_expert && (size_t)T * sh.E * 4 < ((size_t)1 << 32);
+    GroupedArgs ga {};
+    ga.items = b.items; ga.expert_n = b.expert_n; ga.off_pad = b.off_pad; ga.tok_of_q = b.tok_of_q;
+    if (grouped) {
+        __half * rows = (__half *)b.out_pair;        // nothing else is in the pairs' rows until the down projection
+        hipLaunchKernelGGL(k_moe_rows, dim3((unsigned)((size_t)((T + 63) / 64) * (sh.E / 32) * 2)), dim3(256), 0, s, a.x.x, sh.E, T, rows);
+        check_launch("moe_rows");
+        ga.w[0] = L.gate.packed; ga.w[1] = L.up.packed; ga.x = rows; ga.h = b.h.x; ga.K = sh.E; ga.N = sh.F;
+    }
     // (measured on the 128-expert shape at 128 rows: the down projection gains a fifth from the smaller
     // workgroups, gate/up - two weight tiles per wave - loses a tenth, so it keeps two tiles)
+#define RK_MOE_GATE_UP(TYPE)                                                                                     \
+    do {                                                                                                         \
+        if (grouped) grouped_gate_up_launch<TYPE>(s, ga, T, sh);                                                  \
+        else hipLaunchKernelGGL((k_moe_gate_up<TYPE, 2>), dim3(gu_blocks), dim3(256), 0, s, a);                   \
+    } while (0)
     switch (L.gate.type) {
-        case WT_MXFP4: hipLaunchKernelGGL((k_moe_gate_up<WT_MXFP4, 2>), dim3(gu_blocks), dim3(256), 0, s, a); break;
-        case WT_Q4_K:  hipLaunchKernelGGL((k_moe_gate_up<WT_Q4_K, 2>), dim3(gu_blocks), dim3(256), 0, s, a); break;
-        case WT_Q5_K:  hipLaunchKernelGGL((k_moe_gate_up<WT_Q5_K, 2>), dim3(gu_blocks), dim3(256), 0, s, a); break;
-        case WT_Q6_K:  hipLaunchKernelGGL((k_moe_gate_up<WT_Q6_K, 2>), dim3(gu_blocks), dim3(256), 0, s, a); break;
-        default:       hipLaunchKernelGGL((k_moe_gate_up<WT_Q8_0, 2>), dim3(gu_blocks), dim3(256), 0, s, a); break;
+        case WT_MXFP4: RK_MOE_GATE_UP(WT_MXFP4); break;
+        case WT_Q4_K:  RK_MOE_GATE_UP(WT_Q4_K); break;
+        case WT_Q5_K:  RK_MOE_GATE_UP(WT_Q5_K); break;
+        case WT_Q6_K:  RK_MOE_GATE_UP(WT_Q6_K); break;
+        default:       RK_MOE_GATE_UP(WT_Q8_0); break;
     }
+#undef RK_MOE_GATE_UP
     check_launch("moe_gate_up");
     if (xn.faithful) {
         // ggml's arithmetic: the hidden rows are converted, in place, for the down projection
@@ -885,10 +1177,12 @@ Slices moe_ffn(hipStream_t s, const MoeLayer & L, const MoeShape & sh, const Act
     a.w0 = L.down.packed; a.w1 = nullptr; a.x = b.h; a.out_pair = b.out_pair; a.K = sh.F; a.N = sh.E;
     // deferred: the rows leave in pair order, so that the norm reads a token's rows without looking up their slots
     a.pair_of_q = defer_combine ? b.pair_of_q : nullptr;
+    ga.w[0] = L.down.packed; ga.w[1] = nullptr; ga.x = b.h.x; ga.out_pair = b.out_pair; ga.pair_of_q = a.pair_of_q; ga.K = sh.F; ga.N = sh.E;
     const unsigned d_blocks = (unsigned)(((size_t)sh.n_expert * (sh.E / 16) + 3) / 4);
 #define RK_MOE_DOWN(TYPE)                                                                                        \
     do {                                                                                                         \
-        if (one_tile) hipLaunchKernelGGL((k_moe_down<TYPE, 1>), dim3(d_blocks), dim3(256), 0, s, a);              \
+        if (grouped) grouped_down_launch<TYPE>(s, ga, T, sh);                                                     \
+        else if (one_tile) hipLaunchKernelGGL((k_moe_down<TYPE, 1>), dim3(d_blocks), dim3(256), 0, s, a);              \
         else hipLaunchKernelGGL((k_moe_down<TYPE, 2>), dim3(d_blocks), dim3(256), 0, s, a);                       \
     } while (0)
     switch (L.down.type) {

@@ -127,3 +127,23 @@ def test_moe_under_the_ggml_arithmetic(tmp_path, key, monkeypatch):
     print("drift %.2e, conversion %.2e" % (drift, conversion), flush=True)
     assert drift < 0.6 * conversion, (drift, conversion)
     eng.close()
+
+
+@pytest.mark.parametrize("n_seq", [4, 9, 33, 65])
+@pytest.mark.parametrize("key", ["mxfp4", "q8_0", "q4_k", "q5_k", "q6_k"])
+def test_grouped_expert_products_give_the_bits_of_the_small_steps(tmp_path, key, n_seq):
+    """Steps with many pairs per expert multiply an expert's rows 64 at a time (sequences of 16 tokens over 16 experts, 4 used:
+    16, 36, 132 and 260 pairs on average, an expert's last tile anywhere); the same sequences one per step take the kernels
+    for few pairs. Every sum runs over the same products in the same order, so the logits are equal, not close."""
+    path = tmp_path / "moe.gguf"
+    synth.write_model(path, SHAPES[key], seed=9, device="cpu", std=0.05)
+    eng = E.Engine(path, E.EngineConfig(n_ctx=8192, n_seq_max=80, n_batch=2048, n_ubatch=2048))
+    rng = np.random.default_rng(4)
+    prompts = [rng.integers(0, 1024, 16) for _ in range(n_seq)]
+    many = eng.step_logits([(i, p, 0) for i, p in enumerate(prompts)], [(i, j) for i in range(n_seq) for j in (0, 15)])
+    for i in range(n_seq):
+        eng.seq_rm(i)
+    few = np.concatenate([eng.step_logits([(i, p, 0)], [(0, 0), (0, 15)]) for i, p in enumerate(prompts)])
+    assert np.isfinite(many).all()
+    assert np.array_equal(many, few)
+    eng.close()
