@@ -1263,7 +1263,8 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
         n_out = (int)n_want;
     }
     int n_tiles = 0, n_items = 0;
-    if (!stack_) rk::count_attention_work(hd, (int)n_rows, qt_, hp_.n_head_kv, &n_tiles, &n_items, &pk_.split_pages);
+    const int qt = stack_ || decode_in_one_launch((size_t)T == n_rows) ? 0 : qt_;        // (that launch needs no tiles and items)
+    if (qt > 0) rk::count_attention_work(hd, (int)n_rows, qt, hp_.n_head_kv, &n_tiles, &n_items, &pk_.split_pages);
 
     if ((size_t)n_items * 32 > item_meta_.bytes) item_meta_.ensure((size_t)n_items * 48);      // some room to grow into
     pk_.item_a = item_meta_.as<int4>();
@@ -1272,10 +1273,10 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
     try {
         hip_check(hipMemcpyAsync(d_stage_.ptr, h_stage_.ptr, stage_bytes, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync");
         const size_t pt_pack = prof_begin(PC_PACK);
-        rk::pack_step(stream_, d_stage_.as<rk::RowDesc>(), (int)n_rows,
+        rk::pack_step(stream_, d_stage_.as<rk::RowDesc>(), (int)n_rows, T,
                       (const int32_t *)((const uint8_t *)d_stage_.ptr + off_tok),
                       (const rk::TableUpdate *)((const uint8_t *)d_stage_.ptr + off_upd), (int)n_upd,
-                      table_.as<int32_t>(), max_pages_, qt_, hp_.n_head_kv, inv_freq_.as<double>(),
+                      table_.as<int32_t>(), max_pages_, qt, hp_.n_head_kv, inv_freq_.as<double>(),
                       hp_.rope_dim / 2, pk_);
         prof_end(PC_PACK, pt_pack);
         if (n_want > 0)
@@ -1441,10 +1442,22 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
     return 0;
 }
 
+rk::AttnShape Engine::attn_shape() const {
+    const HParams & h = hp_;
+    return rk::AttnShape{h.n_head, h.n_head_kv, h.head_dim, h.rope_dim, h.rope_neox, h.eps, kv_strides_.page, kv_strides_.head, kv_q8_, kv_q8_ != rk::KV_F16 && ggml_activations_};
+}
+
+// Every row decodes one token over an f16 cache in the exact arithmetic: rotation, KV store, attention and split merge
+// are one launch (the output projection's plain activation planes are all it writes).
+bool Engine::decode_in_one_launch(bool one_token_rows) const {
+    return one_token_rows && fused_decode_attention_ && !ggml_activations_ && rk::attention_decode_can(attn_shape(), step_max_resident_);
+}
+
 void Engine::forward(int T, int n_out, int n_tiles, int n_items, bool one_token_rows, bool routed) {
     const HParams & h = hp_;
     const int E = h.n_embd, QD = h.n_head * h.head_dim, KD = h.n_head_kv * h.head_dim, F = h.n_ff;
-    rk::AttnShape sh{h.n_head, h.n_head_kv, h.head_dim, h.rope_dim, h.rope_neox, h.eps, kv_strides_.page, kv_strides_.head, kv_q8_, kv_q8_ != rk::KV_F16 && ggml_activations_};
+    const rk::AttnShape sh = attn_shape();
+    const bool fused_decode = decode_in_one_launch(one_token_rows);
     // The versions of a row its consumers need: the values themselves for F32 / F16 / BF16 weights, the
     // expert router and LoRA factors (`plain`); the converted row for the quantised weights.
     const bool faithful = ggml_activations_;
@@ -1562,10 +1575,6 @@ void Engine::forward(int T, int n_out, int n_tiles, int n_items, bool one_token_
             }
             prof_end(PC_QKV, pt_);
         }
-        // every row decodes one token over an f16 cache in the exact arithmetic: rotation, KV store, attention and
-        // split merge are one launch (the output projection's plain activation planes are all it writes)
-        const bool fused_decode = one_token_rows && fused_decode_attention_ && !faithful
-                                  && rk::attention_decode_can(sh, step_max_resident_);
         size_t pt_;
         if (fused_decode) {
             unsigned long long * stamps = nullptr;

@@ -327,6 +327,8 @@ private:
     void copy_page(int32_t src, int32_t dst);
     void set_page(int32_t slot, int idx, int32_t page);
     void clear_slot(Slot & s, int32_t slot);
+    rk::AttnShape attn_shape() const;
+    bool decode_in_one_launch(bool one_token_rows) const;
     void forward(int T, int n_out, int n_tiles, int n_items, bool one_token_rows, bool routed);
     int run_step(const retro_step_row_v2 * rows2, const retro_step_row * rows1, size_t n_rows,
                  retro_step_out_row_v2 * out2, retro_step_out_row * out1,

@@ -1344,7 +1344,11 @@ __device__ int block_scan_incl(int v, int * scratch) {
     return v;
 }
 
-__global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows, int n_rows,
+// Workgroup 0 plans the step; the others fill its rotation table, which only needs the rows. (In one workgroup the
+// table, a double-precision sine and cosine per token and pair, was most of a decode step's launch: 256 rows of 64
+// pairs 58 -> 17 us, one row 12.4 -> 6.4, with the attention items that such a step does not use left out as well.)
+constexpr int PACK_PAIRS = 2048;        // pairs of the rotation table per workgroup
+__global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows, int n_rows, int T,
                                                const int32_t * __restrict__ toks,
                                                const TableUpdate * __restrict__ upd, int n_upd,
                                                int32_t * __restrict__ table, int max_pages,
@@ -1354,7 +1358,29 @@ __global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows
     __shared__ int carry[3];
     __shared__ int len_count[MAX_SPLIT_PAGES + 1], len_base[MAX_SPLIT_PAGES + 1];
     __shared__ int row_len[1024];
-    __shared__ int long_rows[1024], long_out[1024], n_long;      // rows whose tokens the whole workgroup writes
+    __shared__ int long_rows[1024], long_out[1024], n_long;      // rows whose tokens a wave each writes
+    if (blockIdx.x > 0) {
+        // rotary table of the step: angle = pos * inv_freq[j] in double; inv_freq[pairs] is the magnitude factor of the
+        // rotation (1 unless the model's frequency scaling rule asks for another)
+        const double magnitude = inv_freq[pairs];
+        const int end = min((int)blockIdx.x * PACK_PAIRS, T * pairs);
+        for (int i = ((int)blockIdx.x - 1) * PACK_PAIRS + threadIdx.x; i < end; i += 1024) {
+            const int t = i / pairs, j = i % pairs;
+            // position of token t: from its row (a binary search over tok_off, unless every row is one token)
+            int lo = 0, hi = n_rows - 1;
+            if (T == n_rows) lo = hi = t;
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (rows[mid].tok_off <= t) lo = mid; else hi = mid - 1;
+            }
+            const double ang = (double)(rows[lo].pos0 + (t - rows[lo].tok_off)) * inv_freq[j];
+            double sv, cv;
+            sincos(ang, &sv, &cv);
+            o.rope_cos[i] = (float)(cv * magnitude);
+            o.rope_sin[i] = (float)(sv * magnitude);
+        }
+        return;
+    }
     for (int i = threadIdx.x; i < n_upd; i += 1024) table[(size_t)upd[i].slot * max_pages + upd[i].index] = upd[i].page;
     if (threadIdx.x == 0) { carry[0] = 0; carry[1] = 0; carry[2] = 0; }
     __syncthreads();
@@ -1420,9 +1446,11 @@ __global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows
             }
         }
         __syncthreads();
-        for (int k = 0; k < n_long; ++k) {
+        // a single long row by all sixteen waves, several by a wave each
+        const int share = n_long == 1 ? 1024 : 64, lane = threadIdx.x % share;
+        for (int k = threadIdx.x / share; k < n_long; k += 1024 / share) {
             const RowDesc ld = rows[long_rows[k]];
-            for (int i = threadIdx.x; i < ld.n; i += 1024) write_token(ld, long_rows[k], i, long_out[k]);
+            for (int i = lane; i < ld.n; i += share) write_token(ld, long_rows[k], i, long_out[k]);
         }
         // rows past n_rows contribute zero, so the last thread's inclusive
         // sums are the chunk totals
@@ -1504,32 +1532,14 @@ __global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows
         o.counts[2] = carry[0];
         o.counts[3] = carry[1];
     }
-    // rotary table of the step: angle = pos * inv_freq[j] in double; inv_freq[pairs] is the magnitude factor of the
-    // rotation (1 unless the model's frequency scaling rule asks for another)
-    const double magnitude = inv_freq[pairs];
-    const RowDesc lastd = rows[n_rows - 1];
-    const int T = lastd.tok_off + lastd.n;
-    for (int i = threadIdx.x; i < T * pairs; i += 1024) {
-        const int t = i / pairs, j = i % pairs;
-        // position of token t: recompute from its row (binary search over tok_off)
-        int lo = 0, hi = n_rows - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (rows[mid].tok_off <= t) lo = mid; else hi = mid - 1;
-        }
-        const double ang = (double)(rows[lo].pos0 + (t - rows[lo].tok_off)) * inv_freq[j];
-        double sv, cv;
-        sincos(ang, &sv, &cv);
-        o.rope_cos[i] = (float)(cv * magnitude);
-        o.rope_sin[i] = (float)(sv * magnitude);
-    }
 }
 
-void pack_step(hipStream_t s, const RowDesc * rows, int n_rows, const int32_t * tokens_concat,
+void pack_step(hipStream_t s, const RowDesc * rows, int n_rows, int n_tokens, const int32_t * tokens_concat,
                const TableUpdate * updates, int n_updates, int32_t * table, int max_pages,
                int qt, int n_kv_heads, const double * inv_freq, int rope_pairs, const PackBuffers & out) {
     if (n_rows <= 0) return;
-    hipLaunchKernelGGL(k_pack, dim3(1), dim3(1024), 0, s, rows, n_rows, tokens_concat, updates, n_updates,
+    const int table_wgs = (int)(((size_t)n_tokens * rope_pairs + PACK_PAIRS - 1) / PACK_PAIRS);
+    hipLaunchKernelGGL(k_pack, dim3(1 + table_wgs), dim3(1024), 0, s, rows, n_rows, n_tokens, tokens_concat, updates, n_updates,
                        table, max_pages, qt, n_kv_heads, inv_freq, rope_pairs, out);
     check_launch("pack_step");
 }
