@@ -1211,19 +1211,8 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
 
     // ---- upload the plan and pack it on the device
     const int T = (int)total;
-    const size_t n_upd = pending_updates_.size();
-    const size_t off_tok = n_rows * sizeof(rk::RowDesc);
-    const size_t off_upd = off_tok + (size_t)T * 4;
-    const size_t off_want = off_upd + n_upd * sizeof(rk::TableUpdate);
-    const size_t n_want = want ? want->n : 0;
-    const size_t off_plan = (off_want + n_want * 4 + 15) / 16 * 16;
-    if (stack_) plan_stack(rows, before);
-    const size_t stage_bytes = off_plan + (stack_ ? stack_plan_bytes() : 0);
-    h_stage_.ensure(stage_bytes);
-    d_stage_.ensure(stage_bytes);
-    if (stack_) stage_stack_plan(h_stage_.as<uint8_t>() + off_plan, d_stage_.as<uint8_t>() + off_plan);
-    rk::RowDesc * hd = h_stage_.as<rk::RowDesc>();
-    int32_t * ht = (int32_t *)((uint8_t *)h_stage_.ptr + off_tok);
+    std::vector<rk::RowDesc> & hd = step_descs_;
+    hd.resize(n_rows);
     int n_out = 0;
     bool routed = false;
     step_max_resident_ = 0;
@@ -1244,11 +1233,38 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
                 hd[r].route = 1 + (int32_t)std::distance(row_adapters_.begin(), found);
                 routed = true;
             }
-            std::memcpy(ht + at, row.tokens, (size_t)row.n * 4);
             at += (int)row.n;
             if (row.sample) ++n_out;
         }
     }
+    AttnPlan plan;
+    const int qt = stack_ || decode_in_one_launch((size_t)T == n_rows) ? 0 : qt_;        // (that launch needs no tiles and items)
+    step_wide_.clear();
+    if (qt > 0) {
+        pk_.wide_row = rk::wide_attention_row(hd.data(), (int)n_rows);
+        rk::count_attention_work(hd.data(), (int)n_rows, qt, hp_.n_head_kv, pk_.wide_row, &plan.n_tiles, &plan.n_items, &pk_.split_pages);
+        plan.n_partial = rk::plan_wide_attention(hd.data(), (int)n_rows, hp_.n_head / hp_.n_head_kv, hp_.n_head_kv, pk_.wide_row, !ggml_activations_, plan.n_items, step_wide_);
+        plan.n_wide = (int)step_wide_.size();
+    }
+    const size_t n_upd = pending_updates_.size();
+    const size_t off_tok = n_rows * sizeof(rk::RowDesc);
+    const size_t off_upd = off_tok + (size_t)T * 4;
+    const size_t off_want = off_upd + n_upd * sizeof(rk::TableUpdate);
+    const size_t n_want = want ? want->n : 0;
+    const size_t off_wide = (off_want + n_want * 4 + 15) / 16 * 16;
+    const size_t off_plan = off_wide + step_wide_.size() * sizeof(rk::WideWork);
+    if (stack_) plan_stack(rows, before);
+    const size_t stage_bytes = off_plan + (stack_ ? stack_plan_bytes() : 0);
+    h_stage_.ensure(stage_bytes);
+    d_stage_.ensure(stage_bytes);
+    if (stack_) stage_stack_plan(h_stage_.as<uint8_t>() + off_plan, d_stage_.as<uint8_t>() + off_plan);
+    std::memcpy(h_stage_.ptr, hd.data(), off_tok);
+    {
+        int32_t * ht = (int32_t *)((uint8_t *)h_stage_.ptr + off_tok);
+        for (size_t r = 0; r < n_rows; ++r) std::memcpy(ht + hd[r].tok_off, rows[r].tokens, (size_t)rows[r].n * 4);
+    }
+    if (!step_wide_.empty()) std::memcpy(h_stage_.as<uint8_t>() + off_wide, step_wide_.data(), step_wide_.size() * sizeof(rk::WideWork));
+    plan.wide = (const rk::WideWork *)(d_stage_.as<uint8_t>() + off_wide);
     {
         rk::TableUpdate * hu = (rk::TableUpdate *)((uint8_t *)h_stage_.ptr + off_upd);
         size_t i = 0;
@@ -1262,13 +1278,10 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
         for (size_t i = 0; i < n_want; ++i) hw[i] = hd[want->row[i]].tok_off + (int32_t)want->index[i];
         n_out = (int)n_want;
     }
-    int n_tiles = 0, n_items = 0;
-    const int qt = stack_ || decode_in_one_launch((size_t)T == n_rows) ? 0 : qt_;        // (that launch needs no tiles and items)
-    if (qt > 0) rk::count_attention_work(hd, (int)n_rows, qt, hp_.n_head_kv, &n_tiles, &n_items, &pk_.split_pages);
 
-    if ((size_t)n_items * 32 > item_meta_.bytes) item_meta_.ensure((size_t)n_items * 48);      // some room to grow into
+    if ((size_t)plan.n_items * 32 > item_meta_.bytes) item_meta_.ensure((size_t)plan.n_items * 48);      // some room to grow into
     pk_.item_a = item_meta_.as<int4>();
-    pk_.item_b = pk_.item_a + n_items;
+    pk_.item_b = pk_.item_a + plan.n_items;
 
     try {
         hip_check(hipMemcpyAsync(d_stage_.ptr, h_stage_.ptr, stage_bytes, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync");
@@ -1282,7 +1295,7 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
         if (n_want > 0)
             rk::copy_floats(stream_, (const float *)((const uint8_t *)d_stage_.ptr + off_want), (float *)pk_.out_tok, n_want);
         if (stack_) forward_stack(T, n_out);
-        else forward(T, n_out, n_tiles, n_items, (size_t)T == n_rows, routed);
+        else forward(T, n_out, plan, (size_t)T == n_rows, routed);
         if (want) {
             if (n_want > 0)
                 hip_check(hipMemcpyAsync(want->out, logits_.ptr, n_want * (size_t)n_vocab * 4, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
@@ -1453,7 +1466,7 @@ bool Engine::decode_in_one_launch(bool one_token_rows) const {
     return one_token_rows && fused_decode_attention_ && !ggml_activations_ && rk::attention_decode_can(attn_shape(), step_max_resident_);
 }
 
-void Engine::forward(int T, int n_out, int n_tiles, int n_items, bool one_token_rows, bool routed) {
+void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_rows, bool routed) {
     const HParams & h = hp_;
     const int E = h.n_embd, QD = h.n_head * h.head_dim, KD = h.n_head_kv * h.head_dim, F = h.n_ff;
     const rk::AttnShape sh = attn_shape();
@@ -1516,7 +1529,7 @@ void Engine::forward(int T, int n_out, int n_tiles, int n_items, bool one_token_
         return std::array<int, 3>{t[0], t[1], t[2]};
     };
     const rk::Act act_o = act_for(act_o_x_, act_o_sums_, act_o_qx_, act_o_qsums_, E, {lm_head_.w.type}, false, &act_o_codes_);
-    partial_.ensure(rk::attention_partial_floats(n_items, h.head_dim) * 4);
+    partial_.ensure(rk::attention_partial_floats(plan.n_partial, h.head_dim) * 4);
     float * x = x_.as<float>();
     float * qkv = qkv_.as<float>();
     float * gu = gu_.as<float>();
@@ -1609,12 +1622,15 @@ void Engine::forward(int T, int n_out, int n_tiles, int n_items, bool one_token_
         prof_end(PC_ROPE, pt_);
         pt_ = prof_begin(PC_ATTN);
         rk::attention(stream_, q_half_.as<__half>(), q_half_lo_.as<__half>(), sh, pk_, table_.as<int32_t>(), max_pages_,
-                      k_pool_[(size_t)l].as<__half>(), v_pool_[(size_t)l].as<__half>(), n_items, n_tiles,
+                      k_pool_[(size_t)l].as<__half>(), v_pool_[(size_t)l].as<__half>(), plan.n_items, plan.n_tiles,
                       partial_.as<float>(), one_token_rows);
+        rk::attention_wide(stream_, q_half_.as<__half>(), q_half_lo_.as<__half>(), sh, pk_, table_.as<int32_t>(), max_pages_,
+                           k_pool_[(size_t)l].as<__half>(), v_pool_[(size_t)l].as<__half>(), plan.wide, plan.n_wide,
+                           partial_.as<float>(), act_q);
         prof_end(PC_ATTN, pt_);
         // a single token with few splits: the output projection merges them itself (n_items = kv heads x splits)
-        const int n_split = T == 1 && n_tiles == 1 ? n_items / h.n_head_kv : 0;
-        const bool merge_in_oproj = fuse && n_split >= 1 && n_split <= merge_max_splits_ && n_split * h.n_head_kv == n_items
+        const int n_split = T == 1 && plan.n_tiles == 1 ? plan.n_items / h.n_head_kv : 0;
+        const bool merge_in_oproj = fuse && n_split >= 1 && n_split <= merge_max_splits_ && n_split * h.n_head_kv == plan.n_items
                                     && rk::gemv_can_weight(L.wo.w, 1) && L.wo.w.K == QD && L.wo.w.N == E;
         if (merge_in_oproj) {
             pt_ = prof_begin(PC_OPROJ);
@@ -1624,7 +1640,7 @@ void Engine::forward(int T, int n_out, int n_tiles, int n_items, bool one_token_
             prof_end(PC_OPROJ, pt_);
         } else {
         pt_ = prof_begin(PC_COMBINE);
-        rk::attention_combine(stream_, partial_.as<float>(), T, sh, pk_, act_q);
+        if (plan.n_partial > 0) rk::attention_combine(stream_, partial_.as<float>(), T, sh, pk_, act_q);
         prof_end(PC_COMBINE, pt_);
         pt_ = prof_begin(PC_OPROJ);
         if (fuse_x && rk::gemv_f32_can_weight(L.wo.w, T) && L.wo.w.K == QD && L.wo.w.N == E) {

@@ -327,9 +327,14 @@ private:
     void copy_page(int32_t src, int32_t dst);
     void set_page(int32_t slot, int idx, int32_t page);
     void clear_slot(Slot & s, int32_t slot);
+    // A step's attention launches: tiles and one-wave items of the short rows, the work of the long ones, and the
+    // numbered partial results of both (no pure decode step, which needs none of it).
+    struct AttnPlan { int n_tiles = 0, n_items = 0, n_wide = 0, n_partial = 0; const rk::WideWork * wide = nullptr; };
+    std::vector<rk::RowDesc> step_descs_;
+    std::vector<rk::WideWork> step_wide_;
     rk::AttnShape attn_shape() const;
     bool decode_in_one_launch(bool one_token_rows) const;
-    void forward(int T, int n_out, int n_tiles, int n_items, bool one_token_rows, bool routed);
+    void forward(int T, int n_out, const AttnPlan & plan, bool one_token_rows, bool routed);
     int run_step(const retro_step_row_v2 * rows2, const retro_step_row * rows1, size_t n_rows,
                  retro_step_out_row_v2 * out2, retro_step_out_row * out1,
                  int32_t * out_top_ids, float * out_top_logprobs, size_t n_top_stride, const WantLogits * want);

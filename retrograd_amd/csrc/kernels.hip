@@ -31,6 +31,7 @@
 // result holds rows 4*(l/16)+i, column l%16. Both operands always use the same
 // (lane group, slot) for the same logical k, so the hardware's internal k
 // order never matters.
+#include <algorithm>
 #include <mutex>
 #include <cstdlib>
 #include "dev_common.hpp"
@@ -1402,7 +1403,7 @@ __global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows
         if (threadIdx.x == 0) n_long = 0;
         if (r < n_rows) {
             d = rows[r];
-            tiles = qt > 0 ? (d.n + qt - 1) / qt : 0;
+            tiles = qt > 0 && d.n < o.wide_row ? (d.n + qt - 1) / qt : 0;
             for (int j = 0; j < tiles; ++j) {
                 const int hi = d.pos0 + min(d.n, (j + 1) * qt);
                 items += n_kv * tile_splits(d.kv_begin, hi, o.split_pages);
@@ -1550,7 +1551,7 @@ void pack_step(hipStream_t s, const RowDesc * rows, int n_rows, int n_tokens, co
 // costs the merge kernel a partial result to read, so the largest split that
 // still leaves about a wave per SIMD slot wins, and small steps get the
 // smallest one.
-void count_attention_work(const RowDesc * rows, int n_rows, int qt, int n_kv_heads, int * n_tiles, int * n_items,
+void count_attention_work(const RowDesc * rows, int n_rows, int qt, int n_kv_heads, int wide_row, int * n_tiles, int * n_items,
                           int * split_pages) {
     constexpr int kEnoughItems = 1536;
     int tiles = 0, items = 0, split = MAX_SPLIT_PAGES;
@@ -1558,7 +1559,7 @@ void count_attention_work(const RowDesc * rows, int n_rows, int qt, int n_kv_hea
         tiles = 0; items = 0;
         for (int r = 0; r < n_rows; ++r) {
             const RowDesc & d = rows[r];
-            const int nt = (d.n + qt - 1) / qt;
+            const int nt = d.n < wide_row ? (d.n + qt - 1) / qt : 0;
             for (int j = 0; j < nt; ++j) {
                 const int hi = d.pos0 + std::min(d.n, (j + 1) * qt);
                 const int p_first = d.kv_begin / PAGE, p_last = (hi - 1) / PAGE;
@@ -1571,6 +1572,54 @@ void count_attention_work(const RowDesc * rows, int n_rows, int qt, int n_kv_hea
     *n_tiles = tiles;
     *n_items = items;
     *split_pages = split;
+}
+
+int wide_attention_row(const RowDesc * rows, int n_rows) {
+    constexpr int kRow = 12;
+    constexpr long kPages = 2048;
+    long work = 0;              // pages a wave per token would read
+    for (int r = 0; r < n_rows; ++r)
+        if (rows[r].n >= kRow) work += (long)rows[r].n * ((rows[r].pos0 + rows[r].n - rows[r].kv_begin + PAGE - 1) / PAGE);
+    return work >= kPages ? kRow : INT32_MAX;
+}
+
+int plan_wide_attention(const RowDesc * rows, int n_rows, int G, int n_kv_heads, int wide_row, bool direct, int item0, std::vector<WideWork> & work) {
+    // The longest split that still gives every compute unit two workgroups; a split costs the merge launch a partial
+    // result per token and head, and no split costs no merge at all.
+    constexpr int kEnoughGroups = 512;
+    const int per_tile = wide_tile_tokens(G);
+    auto pages_of = [](int kv_begin, int hi) { return (hi - 1) / PAGE - kv_begin / PAGE + 1; };
+    int split = 1 << 24;
+    for (int s : {1 << 24, 64, 32, 16, 8, 4}) {
+        int groups = 0;
+        for (int r = 0; r < n_rows; ++r) {
+            const RowDesc & d = rows[r];
+            for (int q0 = 0; d.n >= wide_row && q0 < d.n; q0 += per_tile)
+                groups += n_kv_heads * ((pages_of(d.kv_begin, d.pos0 + std::min(d.n, q0 + per_tile)) + s - 1) / s);
+        }
+        split = s;
+        if (groups >= kEnoughGroups || groups == 0) break;
+    }
+    work.clear();
+    int at = item0;
+    for (int r = 0; r < n_rows; ++r) {
+        const RowDesc & d = rows[r];
+        if (d.n < wide_row) continue;
+        for (int q0 = 0; q0 < d.n; q0 += per_tile) {
+            const int nq = std::min(per_tile, d.n - q0);
+            const int pages = pages_of(d.kv_begin, d.pos0 + q0 + nq), first = d.kv_begin / PAGE;
+            const int ns = (pages + split - 1) / split, share = (pages + ns - 1) / ns;
+            const bool alone = ns == 1 && direct;
+            for (int sp = 0; sp < ns; ++sp) {
+                const int lo = sp * share, n = std::max(0, std::min(share, pages - lo));
+                work.push_back({{d.tok_off + q0, nq | (ns << 16), d.pos0 + q0, d.slot}, {d.kv_begin, first + lo, n, alone ? -1 : at + sp}});
+            }
+            if (!alone) at += (nq + 16 / G - 1) / (16 / G) * n_kv_heads * ns;
+        }
+    }
+    // longest first: the tail of the launch is made of short ones
+    std::stable_sort(work.begin(), work.end(), [](const WideWork & a, const WideWork & b) { return a.b.z > b.b.z; });
+    return at;
 }
 
 // ---------------------------------------------------------------------------
@@ -2129,6 +2178,336 @@ __global__ __launch_bounds__(64, 2) void k_attention(AttnArgs a) {
     }
 }
 
+// Rows of many tokens (a portion of a prompt): a workgroup of four waves attends WIDE_CT column tiles per wave, a column
+// being a (token, query head) pair of one kv head and a tile sixteen of them, and every K and V page is staged once for all
+// of them, global -> LDS, the next page while one is multiplied. The hi and the lo half of a query (and of a probability)
+// are two instructions on the same tile. (k_attention, a wave per 8 / G tokens, reads every page once per 8 / G tokens:
+// 1953 tokens after 2048 others, 32 / 8 heads of 128, took 550 us and the merge of its splits 71; this 208, 0.95 PFLOP/s
+// counting both halves, and 40. 2048 tokens after none: 208 + 48 against 102.)
+// What bounds it: the matrix instructions and, nearly as many cycles, the softmax beside them (per score a maximum, an
+// exponential, a sum and the split into halves), over a Q8_0 or Q4_0 cache the widening of codes and scales. PP pages are
+// attended together where registers allow: half the barriers, maxima and exchanges (235 -> 208 us with two).
+constexpr int WIDE_CT = 2;
+int wide_tile_tokens(int G) { return 4 * WIDE_CT * (16 / G); }
+
+struct WideArgs {
+    const __half * q, * q_lo, * k_pool, * v_pool;
+    const int32_t * table;
+    const WideWork * work;
+    float * partial;
+    int4 * tok_merge;
+    Act out;                   // where a tile that is not split leaves its rows
+    int max_pages, n_head, n_kv, G;
+    size_t page_stride, head_stride;
+};
+
+template <int HD, int KVQ, int PP>
+__global__ __launch_bounds__(256, 2) void k_attention_wide(WideArgs a) {
+    constexpr bool Q8 = KVQ != KV_F16;
+    constexpr int KS = HD / 32, DT = HD / 16, CT = WIDE_CT;
+    constexpr int CODES = KVQ == KV_Q8 ? 1024 : KVQ == KV_Q4 ? 512 : 2048;      // bytes of 32 dimensions
+    constexpr int BLOCK = KS * (CODES + (Q8 ? 64 : 0));                          // of a page of one head, K or V
+    __shared__ __attribute__((aligned(16))) uint8_t stage[2][PP][2 * BLOCK];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const WideWork wk = a.work[blockIdx.x / a.n_kv];
+    const int h = blockIdx.x % a.n_kv;
+    const int t0 = __builtin_amdgcn_readfirstlane(wk.a.x), nq = __builtin_amdgcn_readfirstlane(wk.a.y & 0xffff), ns = __builtin_amdgcn_readfirstlane(wk.a.y >> 16);
+    const int pos0 = __builtin_amdgcn_readfirstlane(wk.a.z), slot = __builtin_amdgcn_readfirstlane(wk.a.w), kv_begin = __builtin_amdgcn_readfirstlane(wk.b.x);
+    const int page_first = __builtin_amdgcn_readfirstlane(wk.b.y), n_pages = __builtin_amdgcn_readfirstlane(wk.b.z), item = __builtin_amdgcn_readfirstlane(wk.b.w);
+    const int tpt = 16 / a.G;                       // tokens of a column tile
+    if (h == 0 && page_first == kv_begin / PAGE)    // what the merge launch needs to know of these tokens (no splits: nothing to do)
+        for (int i = threadIdx.x; i < nq; i += 256) a.tok_merge[t0 + i] = make_int4(item + i / tpt * a.n_kv * ns, item < 0 ? 0 : ns, i % tpt, 0);
+    const int QD = a.n_head * HD;
+    const int qi = c / a.G, gi = c % a.G;
+    int tok[CT];
+    bool ok[CT];
+    h8 q_hi[CT][KS], q_lo[CT][KS];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        tok[ct] = (wave * CT + ct) * tpt + qi;
+        ok[ct] = qi < tpt && tok[ct] < nq;
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            q_hi[ct][j] = q_lo[ct][j] = (h8){0, 0, 0, 0, 0, 0, 0, 0};         // (a column without a query: scores of 0, never stored)
+            if (ok[ct]) {
+                const size_t at = (size_t)(t0 + tok[ct]) * QD + (size_t)(h * a.G + gi) * HD + 32 * j + 8 * g;
+                q_hi[ct][j] = load_h8(a.q + at);
+                q_lo[ct][j] = load_h8(a.q_lo + at);
+            }
+        }
+    }
+    // positions of the wave's first and last token: pages behind the last are none of its business, pages that end
+    // before the first need no mask
+    const int w_first = pos0 + wave * CT * tpt, w_last = pos0 + min(nq, (wave + 1) * CT * tpt) - 1;
+    f4 o[CT][DT];
+    float m_run[CT], l_run[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        m_run[ct] = -INFINITY;
+        l_run[ct] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[ct][d] = (f4){0.f, 0.f, 0.f, 0.f};
+    }
+    int my_pid = 0;
+    const uint32_t lds0 = lds_offset(&stage[0][0][0]);
+    auto request = [&](int i, int slot_of) __attribute__((always_inline)) {
+        if ((i & 63) == 0) my_pid = i + lane < n_pages ? a.table[(size_t)slot * a.max_pages + page_first + i + lane] : 0;
+        const int pid = __builtin_amdgcn_readlane(my_pid, i & 63);           // (past the end: page 0, whose scores are masked)
+        // (the requests take their addresses from scalar registers, wherever the compiler has computed them)
+        auto scalar = [](uint64_t v) __attribute__((always_inline)) {
+            return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v)
+                 | ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32);
+        };
+        const size_t at = (size_t)pid * a.page_stride + (size_t)h * a.head_stride;
+        const void * kp = (const void *)scalar((uint64_t)(a.k_pool + at)), * vp = (const void *)scalar((uint64_t)(a.v_pool + at));
+        const uint32_t dst0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + (uint32_t)slot_of * (2 * BLOCK) + (uint32_t)wave * 1024u));
+        constexpr int PIECES = BLOCK / 16;
+#pragma unroll
+        for (int p0 = 0; p0 < PIECES; p0 += 256) {
+            if (p0 + 256 <= PIECES || p0 + (int)threadIdx.x < PIECES) {
+                lds_dma16(kp, (uint32_t)(p0 + threadIdx.x) * 16u, dst0 + p0 * 16u);
+                lds_dma16(vp, (uint32_t)(p0 + threadIdx.x) * 16u, dst0 + p0 * 16u + BLOCK);
+            }
+        }
+    };
+    auto request_group = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < PP; ++u) request(i + u, (i / PP & 1) * PP + u);
+    };
+    const int p_end = (page_first + n_pages) * PAGE - 1;      // the split's last position
+    if (n_pages > 0) request_group(0);
+#pragma unroll 1
+    for (int i = 0; i < n_pages; i += PP) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();                   // the group's pages have landed; none still reads the other buffer
+        if (i + PP < n_pages) request_group(i + PP);
+        __builtin_amdgcn_sched_barrier(0);
+        const int p_lo = (page_first + i) * PAGE;
+        if (p_lo > w_last || w_first > w_last) continue;
+        f4 s[PP][CT][2];
+#pragma unroll
+        for (int u = 0; u < PP; ++u)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) s[u][ct][0] = s[u][ct][1] = (f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < PP; ++u) {
+            const uint8_t * kb = stage[i / PP & 1][u];
+#pragma unroll
+            for (int j = 0; j < KS; ++j) {
+                h8 k0, k1;
+                if constexpr (KVQ == KV_Q8) {
+                    const u4 raw = *(const u4 *)(kb + j * 1024 + lane * 16);
+                    k0 = codes8(raw.x, raw.y);
+                    k1 = codes8(raw.z, raw.w);
+                } else if constexpr (KVQ == KV_Q4) {
+                    const kv_u2 raw = *(const kv_u2 *)(kb + j * 512 + lane * 8);
+                    k0 = codes4(raw.x);
+                    k1 = codes4(raw.y);
+                } else {
+                    k0 = *(const h8 *)(kb + (j * 2) * 1024 + lane * 16);
+                    k1 = *(const h8 *)(kb + (j * 2 + 1) * 1024 + lane * 16);
+                }
+                if constexpr (Q8) {
+                    const h8 dk = *(const h8 *)(kb + KS * CODES + (j * 4 + g) * 16);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        const f4 zero = (f4){0.f, 0.f, 0.f, 0.f};
+                        f4 u0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, q_hi[ct][j], zero, 0, 0, 0);
+                        f4 u1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, q_hi[ct][j], zero, 0, 0, 0);
+                        u0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, q_lo[ct][j], u0, 0, 0, 0);
+                        u1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, q_lo[ct][j], u1, 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            s[u][ct][0][e] = fmaf((float)dk[e], u0[e], s[u][ct][0][e]);
+                            s[u][ct][1][e] = fmaf((float)dk[4 + e], u1[e], s[u][ct][1][e]);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        s[u][ct][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, q_hi[ct][j], s[u][ct][0], 0, 0, 0);
+                        s[u][ct][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, q_hi[ct][j], s[u][ct][1], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        s[u][ct][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, q_lo[ct][j], s[u][ct][0], 0, 0, 0);
+                        s[u][ct][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, q_lo[ct][j], s[u][ct][1], 0, 0, 0);
+                    }
+                }
+            }
+        }
+        // rows of s[u][.][0] are tokens 4 g + e of page u of the group, of s[u][.][1] tokens 16 + 4 g + e
+        const bool edge = p_lo + PP * PAGE - 1 > min(w_first, p_end) || p_lo < kv_begin;
+        float e8[PP][CT][8];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            if (edge) {
+                const int limit = min(pos0 + tok[ct], p_end);
+#pragma unroll
+                for (int u = 0; u < PP; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int p0 = p_lo + u * PAGE + 4 * g + e, p1 = p0 + 16;
+                        if (p0 < kv_begin || p0 > limit) s[u][ct][0][e] = -INFINITY;
+                        if (p1 < kv_begin || p1 > limit) s[u][ct][1][e] = -INFINITY;
+                    }
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int u = 0; u < PP; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fmaxf(s[u][ct][0][e], s[u][ct][1][e]));
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float m_new = fmaxf(m_run[ct], mx);
+            const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+            const float alpha = __builtin_amdgcn_exp2f(m_run[ct] - m_use);       // m_run = -inf -> 0
+            m_run[ct] = m_new;
+            float psum = 0.0f;
+#pragma unroll
+            for (int u = 0; u < PP; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    e8[u][ct][e] = __builtin_amdgcn_exp2f(s[u][ct][0][e] - m_use);
+                    e8[u][ct][4 + e] = __builtin_amdgcn_exp2f(s[u][ct][1][e] - m_use);
+                    psum += e8[u][ct][e] + e8[u][ct][4 + e];
+                }
+            // the running maximum rarely moves after the first pages: then every column's factor is exactly one
+            if (__any(alpha != 1.0f)) {
+                l_run[ct] *= alpha;
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[ct][d][e] *= alpha;
+            }
+            l_run[ct] += psum;
+        }
+#pragma unroll
+        for (int u = 0; u < PP; ++u) {
+            const uint8_t * vb = stage[i / PP & 1][u] + BLOCK;
+            h8 p_hi[CT], p_lw[CT];
+            auto operand = [&](int ct, h8 dv) __attribute__((always_inline)) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float p = Q8 ? e8[u][ct][e] * (float)dv[e] : e8[u][ct][e];
+                    const _Float16 hi = (_Float16)p;
+                    p_hi[ct][e] = hi;
+                    p_lw[ct][e] = (_Float16)(p - (float)hi);
+                }
+            };
+            if constexpr (!Q8) {
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) operand(ct, h8{});
+            }
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                h8 vd;
+                if constexpr (Q8) {
+                    const int b = d >> 1;
+                    if ((d & 1) == 0) {
+                        const h8 dv = *(const h8 *)(vb + KS * CODES + (b * 4 + g) * 16);
+#pragma unroll
+                        for (int ct = 0; ct < CT; ++ct) operand(ct, dv);
+                    }
+                    if constexpr (KVQ == KV_Q8) {
+                        const kv_u2 raw = *(const kv_u2 *)(vb + b * 1024 + lane * 16 + (d & 1) * 8);
+                        vd = codes8(raw.x, raw.y);
+                    } else {
+                        vd = codes4(*(const uint32_t *)(vb + b * 512 + lane * 8 + (d & 1) * 4));
+                    }
+                } else {
+                    vd = *(const h8 *)(vb + d * 1024 + lane * 16);
+                }
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) o[ct][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vd, p_hi[ct], o[ct][d], 0, 0, 0);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) o[ct][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vd, p_lw[ct], o[ct][d], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        float L = l_run[ct];
+        L += __shfl_xor(L, 16, 64);
+        L += __shfl_xor(L, 32, 64);
+        if (item >= 0) {
+            if (!ok[ct]) continue;
+            float * dst = a.partial + ((size_t)(item + ((wave * CT + ct) * a.n_kv + h) * ns) * 16 + c) * (HD + 2);
+            if (g == 0) { dst[0] = m_run[ct]; dst[1] = L; }
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dst[2 + d * 16 + 4 * g + e] = o[ct][d][e];
+            continue;
+        }
+        // not split: the output projection's activations, as k_attention_combine stores them (the lanes of a column are
+        // here together, with or without a query)
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        const int t = t0 + tok[ct];
+#pragma unroll
+        for (int b = 0; b < KS; ++b) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+                h4 hi, lo;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v = fminf(fmaxf(o[ct][2 * b + u][e] * inv, -65504.0f), 65504.0f);
+                    hi[e] = (_Float16)v;
+                    lo[e] = (_Float16)(v - (float)hi[e]);
+                    sum += (float)hi[e] + (float)lo[e];
+                }
+                if (ok[ct]) {
+                    const int k = (h * a.G + gi) * HD + (2 * b + u) * 16 + 4 * g;
+                    *(h4 *)(a.out.x + act_at(t, k, 0, QD)) = hi;
+                    *(h4 *)(a.out.x + act_at(t, k, 1, QD)) = lo;
+                }
+            }
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            if (ok[ct] && g == 0 && a.out.sums) {
+                const int blk = ((h * a.G + gi) * HD) / 32 + b;
+                const __half s_hi = sat_half(sum);
+                a.out.sums[act_sum_at(t, blk, 0, QD)] = s_hi;
+                a.out.sums[act_sum_at(t, blk, 1, QD)] = __float2half_rn(sum - __half2float(s_hi));
+            }
+        }
+    }
+}
+
+void attention_wide(hipStream_t s, const __half * q, const __half * q_lo, const AttnShape & sh, const PackBuffers & pk,
+                    const int32_t * table, int max_pages, const __half * k_pool, const __half * v_pool, const WideWork * work,
+                    int n_work, float * partial, const Act & out) {
+    if (n_work <= 0) return;
+    const int G = sh.n_head_kv > 0 ? sh.n_head / sh.n_head_kv : 0;
+    if (G < 1 || G > 16 || sh.n_head % sh.n_head_kv != 0) throw std::runtime_error("attention: unsupported head grouping");
+    if (sh.page_stride == 0 || sh.head_stride == 0) throw std::runtime_error("attention: the pool's strides are missing");
+    if (!out.faithful && !out.x) throw std::runtime_error("attention: the output projection's activations are missing");
+    WideArgs a {};
+    a.q = q; a.q_lo = q_lo; a.k_pool = k_pool; a.v_pool = v_pool; a.table = table; a.work = work; a.partial = partial;
+    a.tok_merge = pk.tok_merge; a.out = out; a.max_pages = max_pages;
+    a.n_head = sh.n_head; a.n_kv = sh.n_head_kv; a.G = G;
+    a.page_stride = sh.page_stride; a.head_stride = sh.head_stride;
+    const dim3 grid((unsigned)n_work * (unsigned)sh.n_head_kv), block(256);
+#define ATTN_WIDE(HD_) \
+    do { \
+        if (sh.kv_quant == KV_Q8) hipLaunchKernelGGL((k_attention_wide<HD_, KV_Q8, 1>), grid, block, 0, s, a); \
+        else if (sh.kv_quant == KV_Q4) hipLaunchKernelGGL((k_attention_wide<HD_, KV_Q4, 1>), grid, block, 0, s, a); \
+        else if (sh.kv_quant == KV_F16) hipLaunchKernelGGL((k_attention_wide<HD_, KV_F16, 2>), grid, block, 0, s, a); \
+        else throw std::runtime_error("attention: unknown cache type"); \
+    } while (0)
+    switch (sh.head_dim) {
+        case 32:  ATTN_WIDE(32); break;
+        case 64:  ATTN_WIDE(64); break;
+        case 128: ATTN_WIDE(128); break;
+        default: throw std::runtime_error("attention: head_dim must be 32, 64 or 128");
+    }
+#undef ATTN_WIDE
+    check_launch("attention_wide");
+}
+
 size_t attention_partial_floats(int n_items, int head_dim) {
     return (size_t)n_items * 16 * (head_dim + 2);
 }
@@ -2187,11 +2566,12 @@ __global__ __launch_bounds__(256) void k_attention_combine(CombineArgs a) {
     const int wave = threadIdx.x >> 6;
     const int head = blockIdx.y * 4 + wave;
     const int lane = threadIdx.x & 63;
+    const int4 meta = a.tok_merge[t];            // first item of the token's tile, splits, index in the tile
+    if (meta.y == 0) return;                     // k_attention_wide has left its rows already
     const bool live = head < a.n_head;           // a wave without a head still meets the others at the barrier
     const int e0 = 2 * lane;
     float M = -INFINITY, L = 0.0f, v0 = 0.0f, v1 = 0.0f;
     if (live) {
-        const int4 meta = a.tok_merge[t];                  // first item of the token's tile, splits, index in the tile
         const int ns = meta.y;
         const int kvh = head / a.G, gi = head % a.G;
         const int col = meta.z * a.G + gi;

@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 namespace rk {
 
@@ -351,6 +352,7 @@ struct PackBuffers {       // device arrays, sized for n_batch tokens / rows
     int32_t * dec_pid;     // [n_rows][8] in that order: with the row's pages dealt evenly to eight waves, the id of each wave's first page
     float * rope_cos;      // [T][rope_dim/2]
     float * rope_sin;
+    int wide_row = INT32_MAX;            // rows of at least this many tokens have no tiles and items (set from wide_attention_row)
     int split_pages = MAX_SPLIT_PAGES;   // pages per attention work item in this step (set from count_attention_work)
 };
 // Applies the block-table updates, then derives every per-token / per-tile
@@ -364,8 +366,22 @@ void pack_step(hipStream_t s, const RowDesc * rows, int n_rows, int n_tokens, co
 // Query tokens per attention tile for G query heads per kv head: 8 / G when the hi and lo halves of a query
 // share a matrix instruction (G <= 8), else 16 / G.
 inline int attention_tile_tokens(int G) { return G <= 8 ? 8 / G : (16 / G > 0 ? 16 / G : 1); }
+// Rows of at least this many tokens are attended by attention_wide in this step; k_pack plans tiles and items for the others.
+// Short rows waste its columns and little work its workgroups: with rows of 12 and more tokens and 2048 pages times tokens it
+// is the faster launch (us per layer with the merge, one-wave items / wide, 32 / 8 heads of 128: 4 rows of 16, 24, 63 tokens at
+// position 600 19.8 / 20.7, 23.7 / 23.1, 39.5 / 34.4; 24 rows of 8, 12, 24, 63 36.8 / 37.5, 46.6 / 44.5, 69.6 / 57.6, 145 / 90).
+int wide_attention_row(const RowDesc * rows, int n_rows);
+// One workgroup per kv head: a = {first flat token, tokens | splits << 16, position of the first token, slot},
+// b = {first resident position of the slot, first page of the split, its pages, number of the tile's first work item plus the
+// split - or -1: not split, the rows leave as the output projection's activations}. The items of a tile of
+// wide_tile_tokens are numbered [column tile of 16 / G tokens][kv head][split].
+struct WideWork { int4 a, b; };
+int wide_tile_tokens(int G);
+// The step's work over its long rows; item numbers start at item0, `direct`: tiles that are not split leave their rows
+// themselves. Returns the number behind the last item.
+int plan_wide_attention(const RowDesc * rows, int n_rows, int G, int n_kv_heads, int wide_row, bool direct, int item0, std::vector<WideWork> & work);
 // Host mirror of the tile/item count (same formula as the kernel).
-void count_attention_work(const RowDesc * rows, int n_rows, int qt, int n_kv_heads,
+void count_attention_work(const RowDesc * rows, int n_rows, int qt, int n_kv_heads, int wide_row,
                           int * n_tiles, int * n_items, int * split_pages);
 
 // ---- attention ----------------------------------------------------------------
@@ -436,6 +452,11 @@ void attention_decode(hipStream_t s, const float * qkv, const Slices & from, int
                       const float * q_norm, const float * k_norm, const Act & out, unsigned long long * stamps = nullptr);
 void attention_combine(hipStream_t s, const float * partial, int T, const AttnShape & sh,
                        const PackBuffers & pk, const Act & out);
+// Paged attention of the step's long rows (work on the device, n_work entries); tiles that are split leave partial
+// results for attention_combine, the others their activations in `out`.
+void attention_wide(hipStream_t s, const __half * q, const __half * q_lo, const AttnShape & sh, const PackBuffers & pk,
+                    const int32_t * table, int max_pages, const __half * k_pool, const __half * v_pool, const WideWork * work,
+                    int n_work, float * partial, const Act & out);
 size_t attention_partial_floats(int n_items, int head_dim);
 
 // Gathers the K or V row of one (layer pool, cell) into natural order, and the
