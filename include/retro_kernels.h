@@ -164,6 +164,12 @@ int retro_engine_debug_single_token_matvec(retro_engine * engine, int32_t enable
 int retro_engine_step_logits(retro_engine * engine, const retro_step_row_v2 * rows, size_t n_rows,
                              const uint32_t * want_row, const uint32_t * want_index, size_t n_want, float * out_logits);
 
+/* Page-locked host memory for results: a device copy into it is one transfer (into ordinary memory it is staged, and
+ * fresh pages fault). NULL when the machine gives none; free accepts NULL. Usable from every thread and device, and
+ * independent of any engine's life. */
+void * retro_host_alloc(size_t n_bytes);
+void retro_host_free(void * ptr);
+
 /* Layer-stack models: while on, every step keeps the residual stream after each layer; read copies the last step's,
  * [layer][token][width] (out = NULL: only the number of tokens). */
 int retro_engine_debug_keep_residual(retro_engine * engine, bool on);

@@ -207,6 +207,19 @@ int retro_engine_step_logits(retro_engine * engine, const retro_step_row_v2 * ro
     });
 }
 
+void * retro_host_alloc(size_t n_bytes) {
+    void * ptr = nullptr;
+    if (n_bytes == 0 || hipHostMalloc(&ptr, n_bytes, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return ptr;
+}
+
+void retro_host_free(void * ptr) {
+    if (ptr) (void)hipHostFree(ptr);
+}
+
 int retro_engine_debug_keep_residual(retro_engine * engine, bool on) {
     return boundary([&]() -> int {
         Engine * e = checked(engine);
