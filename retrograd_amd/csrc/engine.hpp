@@ -383,7 +383,7 @@ private:
     float * last_token_ = nullptr;          // of every slot, in two planes
     DevBuf st_h_, st_proj_, st_cq_, st_q_, st_qa_, st_ol_, st_mix_, st_ff_, st_out_, st_partial_, st_xbc_, st_y_;
     DevBuf st_beside_, st_in_rows_;         // Mamba-2 beside attention; a sublayer's input rows before their convolution
-    DevBuf st_first_, st_low_, st_decay_, st_chunks_;      // values of the first layer that mixes them; the delta rule's
+    DevBuf st_first_, st_low_, st_decay_, st_chunks_;      // values of the first layer that mixes them; of the chunks of recurrent mixers: the delta rule's
     DevBuf st_embed_, st_rows_, st_route_, ex_sel_, ex_weight_, ex_slot_, ex_tiles_, ex_h_;
     int st_proj_ld_ = 0;
     struct BlockPlan { int heads, cols; size_t first, n; };    // attention blocks of the step for one number of query columns per token

@@ -550,6 +550,7 @@ void Engine::build_stack() {
         if (sp.state_space()) {
             xbc = std::max(xbc, (size_t)B * sp.mamba.channels());
             y = std::max(y, (size_t)B * sp.mamba.inner());
+            chunks = std::max(chunks, rk::mamba_chunk_floats(sp.mamba, B));
             if (sp.beside_width() > 0) beside = std::max(beside, rk::frag_elems(B, rk::frags_of(sp.beside_width())));
         }
         if (sp.moe.experts > 0) {
@@ -770,7 +771,7 @@ void Engine::mix_mamba(const StackLayer & L, const StackRun & run, int T, void *
     j.eps = stack_->eps;
     j.runs = step_runs();
     j.conv_state = run.conv_state; j.conv_plane = conv_plane_floats_; j.state = run.state;
-    j.xbc = st_xbc_.as<float>(); j.y = st_y_.as<float>();
+    j.xbc = st_xbc_.as<float>(); j.y = st_y_.as<float>(); j.chunks = st_chunks_.as<float>();
     j.out = out; j.out_kf = rk::frags_of(L.spec.mamba.inner());
     rk::mamba_mix(stream_, arith_, j, T);
     prof_end(PC_SCAN, pt);

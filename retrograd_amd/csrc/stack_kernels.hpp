@@ -328,9 +328,12 @@ struct MambaJob {
     float * state = nullptr;       // [slots][heads][state][vdim]
     float * xbc = nullptr;         // scratch [T][channels]
     float * y = nullptr;           // scratch [T][inner]
+    float * chunks = nullptr;      // scratch of mamba_chunk_floats(sh, T)
+    float * chunk_decay = nullptr; // behind the chunks' states (set by mamba_mix)
     void * out = nullptr;          // activations, inner wide
     int out_kf = 0;
 };
+size_t mamba_chunk_floats(const MambaShape & sh, int T);
 void mamba_mix(hipStream_t s, int arith, const MambaJob & j, int T);
 
 // ---- matrix states with a rule of writing: gated delta rules, linear attention with a forget gate -------------

@@ -224,6 +224,30 @@ def test_recurrence_of_unusual_sizes(tmp_path, kv):
         close(feed(eng, 1, toks, [70, 63, 1, 2, 40, 1]), want, kv)
 
 
+@pytest.mark.parametrize("kv", KINDS)
+@pytest.mark.parametrize("shape", [(16, 64, 128, 2), (3, 100, 20, 1), (4, 30, 50, 4), (2, 5, 3, 1)], ids=lambda s: "x".join(map(str, s)))
+def test_runs_of_every_length_beside_each_other(tmp_path, shape, kv):
+    """One step with runs on both sides of the chunked form's least length and of one, two and more chunks, on fresh and on
+    continued states, and the step after it: every sequence as if it were alone."""
+    heads, vdim, state, groups = shape
+    m = Model(tmp_path / "runs", Y.dibosun(72, 50, [Y.mamba2_layer(heads=heads, vdim=vdim, state=state, groups=groups, conv=4, norm_groups=1, ff=0)] * 2))
+    lens = [1, 129, 31, 32, 2, 33, 64, 65, 128]
+    toks = [m.tokens(n + 43, 100 + n) for n in lens]
+    with m.engine(kv, n_ctx=1024, n_batch=512, slots=len(lens)) as eng:
+        at = [0] * len(lens)
+        got = [[] for _ in lens]
+        for step in ([40 if k % 2 else 0 for k in range(len(lens))], lens, [3 if k % 2 else 43 for k in range(len(lens))]):
+            rows = [(k, toks[k][at[k]:at[k] + n], at[k]) for k, n in enumerate(step) if n]
+            out = eng.step_logits(rows, [(r, i) for r, row in enumerate(rows) for i in range(len(row[1]))])
+            for k, t, _ in rows:
+                got[k].append(out[:len(t)])
+                out = out[len(t):]
+                at[k] += len(t)
+        for k, t in enumerate(toks):
+            assert at[k] == len(t)
+            close(np.concatenate(got[k]), m.plain(t), kv, lens[k])
+
+
 def sharpen(cfg, tensors):
     """Queries of every head point at the keys that token 7 leaves, far above all others."""
     m = cfg["layers"][0]["mixer"]
