@@ -1224,7 +1224,7 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
             hd[r].sample = row.sample ? 1 : 0; hd[r].kv_begin = slots_[(size_t)row.slot].begin;
             step_max_resident_ = std::max(step_max_resident_, row.pos0 + (int32_t)row.n - hd[r].kv_begin);
             // route = 1-based index of the adapter in id order (0: the base model)
-            hd[r].route = 0; hd[r].pad = 0;
+            hd[r].route = 0; hd[r].shared = 0;
             // adapter 0 follows the context: its default adapter, else the trained adapter when there is one
             int32_t eff = row.adapter;
             if (eff == 0) eff = default_adapter_ != 0 ? default_adapter_ : kPolicyAdapter;
@@ -1244,6 +1244,11 @@ int Engine::run_step(const retro_step_row_v2 * rows2, const retro_step_row * row
         pk_.wide_row = rk::wide_attention_row(hd.data(), (int)n_rows);
         rk::count_attention_work(hd.data(), (int)n_rows, qt, hp_.n_head_kv, pk_.wide_row, &plan.n_tiles, &plan.n_items, &pk_.split_pages);
         plan.n_partial = rk::plan_wide_attention(hd.data(), (int)n_rows, hp_.n_head / hp_.n_head_kv, hp_.n_head_kv, pk_.wide_row, !ggml_activations_, plan.n_items, step_wide_);
+        plan.n_wide = (int)step_wide_.size();
+    } else if (!stack_ && n_rows > 1) {
+        step_pages_.resize(n_rows);
+        for (size_t r = 0; r < n_rows; ++r) step_pages_[r] = slots_[(size_t)rows[r].slot].pages.data();
+        plan.n_partial = rk::plan_shared_pages(hd.data(), (int)n_rows, step_pages_.data(), hp_.n_head / hp_.n_head_kv, hp_.n_head_kv, step_wide_);
         plan.n_wide = (int)step_wide_.size();
     }
     const size_t n_upd = pending_updates_.size();
@@ -1596,10 +1601,22 @@ void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_row
                 attn_stamps_.ensure(attn_stamped_wgs_ * 6 * sizeof(unsigned long long));
                 stamps = attn_stamps_.as<unsigned long long>();
             }
-            pt_ = prof_begin(PC_ATTN);
-            rk::attention_decode(stream_, qkv, qkv_slices, T, sh, pk_, table_.as<int32_t>(), max_pages_,
-                                 k_pool_[(size_t)l].as<__half>(), v_pool_[(size_t)l].as<__half>(), L.q_norm.as<float>(),
-                                 L.k_norm.as<float>(), act_q, stamps);
+            __half * k_pool = k_pool_[(size_t)l].as<__half>(), * v_pool = v_pool_[(size_t)l].as<__half>();
+            if (plan.n_wide > 0) {          // rows that share pages
+                pt_ = prof_begin(PC_ROPE);
+                rk::rope_store(stream_, qkv, T, sh, pk_, L.q_norm.as<float>(), L.k_norm.as<float>(), q_half_.as<__half>(),
+                               q_half_lo_.as<__half>(), k_pool, v_pool, qkv_slices);
+                prof_end(PC_ROPE, pt_);
+                pt_ = prof_begin(PC_ATTN);
+                rk::attention_wide(stream_, q_half_.as<__half>(), q_half_lo_.as<__half>(), sh, pk_, table_.as<int32_t>(), max_pages_,
+                                   k_pool, v_pool, plan.wide, plan.n_wide, partial_.as<float>(), act_q);
+                rk::attention_tail(stream_, q_half_.as<__half>(), q_half_lo_.as<__half>(), T, sh, pk_, table_.as<int32_t>(), max_pages_,
+                                   k_pool, v_pool, partial_.as<float>(), act_q);
+            } else {
+                pt_ = prof_begin(PC_ATTN);
+                rk::attention_decode(stream_, qkv, qkv_slices, T, sh, pk_, table_.as<int32_t>(), max_pages_, k_pool, v_pool,
+                                     L.q_norm.as<float>(), L.k_norm.as<float>(), act_q, stamps);
+            }
             prof_end(PC_ATTN, pt_);
             pt_ = prof_begin(PC_OPROJ);
             if (fuse_x && rk::gemv_f32_can_weight(L.wo.w, T) && L.wo.w.K == QD && L.wo.w.N == E) {

@@ -332,6 +332,7 @@ private:
     struct AttnPlan { int n_tiles = 0, n_items = 0, n_wide = 0, n_partial = 0; const rk::WideWork * wide = nullptr; };
     std::vector<rk::RowDesc> step_descs_;
     std::vector<rk::WideWork> step_wide_;
+    std::vector<const int32_t *> step_pages_;      // page ids of the rows' slots, while the step is planned
     rk::AttnShape attn_shape() const;
     bool decode_in_one_launch(bool one_token_rows) const;
     void forward(int T, int n_out, const AttnPlan & plan, bool one_token_rows, bool routed);

@@ -1371,6 +1371,8 @@ __device__ int block_scan_incl(int v, int * scratch) {
 // Workgroup 0 plans the step; the others fill its rotation table, which only needs the rows. (In one workgroup the
 // table, a double-precision sine and cosine per token and pair, was most of a decode step's launch: 256 rows of 64
 // pairs 58 -> 17 us, one row 12.4 -> 6.4, with the attention items that such a step does not use left out as well.)
+constexpr int TAIL_SPLITS = 8;          // partial results of shared pages a row merges at most
+constexpr int DEC_SHARED = 30;          // bit of dec_desc's token index: the row has partial results of shared pages
 constexpr int PACK_PAIRS = 2048;        // pairs of the rotation table per workgroup
 __global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows, int n_rows, int T,
                                                const int32_t * __restrict__ toks,
@@ -1530,7 +1532,7 @@ __global__ __launch_bounds__(1024) void k_pack(const RowDesc * __restrict__ rows
     auto describe = [&](int rank, const RowDesc & d) {
         o.dec_order[rank] = d.tok_off;
         const int pos = d.pos0 + d.n - 1;
-        o.dec_desc[rank] = make_int4(d.tok_off + d.n - 1, pos, d.kv_begin, d.slot);
+        o.dec_desc[rank] = make_int4((d.tok_off + d.n - 1) | (d.shared << DEC_SHARED), pos, d.kv_begin, d.slot);
         const int page_first = d.kv_begin / PAGE, n_pages = pos / PAGE - page_first + 1;
         const int per_wave = (n_pages + 7) / 8;
         for (int w = 0; w < 8; ++w)
@@ -1641,6 +1643,67 @@ int plan_wide_attention(const RowDesc * rows, int n_rows, int G, int n_kv_heads,
         }
     }
     // longest first: the tail of the launch is made of short ones
+    std::stable_sort(work.begin(), work.end(), [](const WideWork & a, const WideWork & b) { return a.b.z > b.b.z; });
+    return at;
+}
+
+int plan_shared_pages(RowDesc * rows, int n_rows, const int32_t * const * pages, int G, int n_kv_heads, std::vector<WideWork> & work) {
+    // (kTileRows: a page costs a tile what it costs as many rows of the decode launch)
+    constexpr int kTileRows = 5, kLeastShare = 8, kEnoughGroups = 512;
+    constexpr double kCUs = 256.0;
+    const double rounds = (double)n_rows * n_kv_heads / kCUs;
+    if (G < 1 || G > 16 || rounds < 4.0) return 0;
+    const int per_tile = wide_tile_tokens(G);
+    // full pages of a row (the page of the new position is its own)
+    auto full = [&](int r) { return rows[r].n == 1 && rows[r].kv_begin == 0 ? rows[r].pos0 / PAGE : 0; };
+    std::vector<int> same((size_t)n_rows);      // pages that a row has in common with the one before it
+    double row_pages = 0;
+    for (int r = 0; r < n_rows; ++r) {
+        row_pages += (rows[r].pos0 + rows[r].n - rows[r].kv_begin + PAGE - 1) / PAGE;
+        if (r > 0) same[(size_t)r] = (int)(std::mismatch(pages[r], pages[r] + std::min(full(r - 1), full(r)), pages[r - 1]).first - pages[r]);
+    }
+    struct Tile { int row, n, pages; };
+    std::vector<Tile> tiles;
+    int most_own = 0, tile_pages = 0;
+    for (int r = 0; r < n_rows;) {
+        Tile best{r, 1, 0};
+        long most = 0;
+        for (int n = 2, shared = full(r); n <= per_tile && r + n <= n_rows; ++n) {
+            shared = std::min(shared, same[(size_t)(r + n - 1)]);
+            if (shared == 0) break;
+            const long gain = (long)shared * (n - kTileRows);
+            if (gain > most) { most = gain; best = {r, n, shared}; }
+        }
+        if (best.pages > 0) {
+            tiles.push_back(best);
+            tile_pages += best.pages;
+        }
+        for (int k = r; k < r + best.n; ++k) most_own = std::max(most_own, (rows[k].pos0 - rows[k].kv_begin) / PAGE + 1 - best.pages);
+        r += best.n;
+    }
+    if (tiles.empty()) return 0;
+    // us per layer, measured with 32 / 8 heads of 128, decode launch / rotation, shared and own pages with the gaps between them:
+    // 256 rows with 2048 positions in common and 200 of their own 146 / 76, 512 + 200 86 / 57, 128 + 200 72 / 50, 256 rows in
+    // eights 1000 + 8 118 / 60, 128 rows 2048 + 200 75 / 55, 512 + 200 45 / 49, 64 rows 2048 + 200 40 / 57.
+    const double decode = rounds * (8.0 + 0.16 * row_pages / n_rows);
+    const double apart = 35.0 + 0.5 * rounds + 1.1 * tile_pages * n_kv_heads / kCUs + 1.4 * most_own;
+    if (1.15 * apart >= decode) return 0;
+    const int groups = (int)tiles.size() * n_kv_heads;
+    int at = 0;
+    for (const Tile & t : tiles) {
+        const int want = std::min(TAIL_SPLITS, (kEnoughGroups + groups - 1) / groups);
+        const int ns = std::max(1, std::min(want, t.pages / kLeastShare)), share = (t.pages + ns - 1) / ns;
+        for (int sp = 0; sp < ns; ++sp) {
+            const int lo = sp * share, n = std::max(0, std::min(share, t.pages - lo));
+            // (as tokens of one sequence behind the shared pages: nothing of them is masked)
+            work.push_back({{rows[t.row].tok_off, t.n | (ns << 16), t.pages * PAGE, rows[t.row].slot}, {0, lo, n, at + sp}});
+        }
+        at += (t.n + 16 / G - 1) / (16 / G) * n_kv_heads * ns;
+        for (int r = t.row; r < t.row + t.n; ++r) {
+            rows[r].kv_begin = t.pages * PAGE;
+            rows[r].shared = 1;
+        }
+    }
     std::stable_sort(work.begin(), work.end(), [](const WideWork & a, const WideWork & b) { return a.b.z > b.b.z; });
     return at;
 }
@@ -2201,6 +2264,41 @@ __global__ __launch_bounds__(64, 2) void k_attention(AttnArgs a) {
     }
 }
 
+// An attention output as the output projection's activations, as k_attention_combine stores it: lane (g, column) holds dims
+// 16 d + 4 g + e of its column's head in o[d][e]. The four lanes of a column are here together, with or without a query.
+template <int HD>
+__device__ __forceinline__ void store_columns(const Act & out, const f4 (&o)[HD / 16], float inv, bool ok, int t, int head, int g, int QD) {
+#pragma unroll
+    for (int b = 0; b < HD / 32; ++b) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+            h4 hi, lo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = fminf(fmaxf(o[2 * b + u][e] * inv, -65504.0f), 65504.0f);
+                hi[e] = (_Float16)v;
+                lo[e] = (_Float16)(v - (float)hi[e]);
+                sum += (float)hi[e] + (float)lo[e];
+            }
+            if (ok) {
+                const int k = head * HD + (2 * b + u) * 16 + 4 * g;
+                *(h4 *)(out.x + act_at(t, k, 0, QD)) = hi;
+                *(h4 *)(out.x + act_at(t, k, 1, QD)) = lo;
+            }
+        }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        if (ok && g == 0 && out.sums) {
+            const int blk = head * HD / 32 + b;
+            const __half s_hi = sat_half(sum);
+            out.sums[act_sum_at(t, blk, 0, QD)] = s_hi;
+            out.sums[act_sum_at(t, blk, 1, QD)] = __float2half_rn(sum - __half2float(s_hi));
+        }
+    }
+}
+
 // Rows of many tokens (a portion of a prompt): a workgroup of four waves attends WIDE_CT column tiles per wave, a column
 // being a (token, query head) pair of one kv head and a tile sixteen of them, and every K and V page is staged once for all
 // of them, global -> LDS, the next page while one is multiplied. The hi and the lo half of a query (and of a probability)
@@ -2464,39 +2562,8 @@ __global__ __launch_bounds__(256, 2) void k_attention_wide(WideArgs a) {
                 for (int e = 0; e < 4; ++e) dst[2 + d * 16 + 4 * g + e] = o[ct][d][e];
             continue;
         }
-        // not split: the output projection's activations, as k_attention_combine stores them (the lanes of a column are
-        // here together, with or without a query)
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        const int t = t0 + tok[ct];
-#pragma unroll
-        for (int b = 0; b < KS; ++b) {
-            float sum = 0.0f;
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                h4 hi, lo;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = fminf(fmaxf(o[ct][2 * b + u][e] * inv, -65504.0f), 65504.0f);
-                    hi[e] = (_Float16)v;
-                    lo[e] = (_Float16)(v - (float)hi[e]);
-                    sum += (float)hi[e] + (float)lo[e];
-                }
-                if (ok[ct]) {
-                    const int k = (h * a.G + gi) * HD + (2 * b + u) * 16 + 4 * g;
-                    *(h4 *)(a.out.x + act_at(t, k, 0, QD)) = hi;
-                    *(h4 *)(a.out.x + act_at(t, k, 1, QD)) = lo;
-                }
-            }
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
-            if (ok[ct] && g == 0 && a.out.sums) {
-                const int blk = ((h * a.G + gi) * HD) / 32 + b;
-                const __half s_hi = sat_half(sum);
-                a.out.sums[act_sum_at(t, blk, 0, QD)] = s_hi;
-                a.out.sums[act_sum_at(t, blk, 1, QD)] = __float2half_rn(sum - __half2float(s_hi));
-            }
-        }
+        // not split: the output projection's activations
+        store_columns<HD>(a.out, o[ct], L > 0.0f ? 1.0f / L : 0.0f, ok[ct], t0 + tok[ct], h * a.G + gi, g, QD);
     }
 }
 
@@ -2529,6 +2596,186 @@ void attention_wide(hipStream_t s, const __half * q, const __half * q_lo, const 
     }
 #undef ATTN_WIDE
     check_launch("attention_wide");
+}
+
+struct TailArgs {
+    const __half * q, * q_lo, * k_pool, * v_pool;
+    const int32_t * table;
+    const int4 * desc;         // as of k_attention_decode; bit DEC_SHARED of the token index: tok_merge names partial results
+    const int4 * tok_merge;
+    const float * partial;
+    Act out;
+    int max_pages, n_rows, n_head, n_kv, G;
+    size_t page_stride, head_stride;
+};
+
+// One-token rows that share pages: what is left of them behind k_attention_wide's part. A wave per (row, kv head) with the
+// arithmetic of k_attention_decode's waves: it starts from the partial results of the shared pages, attends the row's own pages
+// (the step's keys and values are in the cache already) and leaves the output projection's activations. The next page's K is
+// requested when the scores are made and its V when the outputs are, into the registers these have left: a wave alone waits
+// for memory, three on a SIMD cover each other.
+template <int HD>
+__global__ __launch_bounds__(256, 2) void k_attention_tail(TailArgs a) {
+    constexpr int KS = HD / 32, DT = HD / 16, PS = HD + 2;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4, cc = c & 7;
+    // (workgroups go to the XCDs in turn: the rows of a kv head, which may share more pages yet, meet in one or few L2s)
+    const int h = blockIdx.x % a.n_kv, row = blockIdx.x / a.n_kv * 4 + wave;
+    if (row >= a.n_rows) return;
+    const int4 dd = a.desc[row];
+    const int t = __builtin_amdgcn_readfirstlane(dd.x & ((1 << DEC_SHARED) - 1)), shared = __builtin_amdgcn_readfirstlane(dd.x >> DEC_SHARED & 1);
+    const int pos = __builtin_amdgcn_readfirstlane(dd.y), kv_begin = __builtin_amdgcn_readfirstlane(dd.z), slot = __builtin_amdgcn_readfirstlane(dd.w);
+    const int page_first = kv_begin / PAGE, n_pages = pos / PAGE - page_first + 1;
+    const bool col_ok = cc < a.G, lo_col = c >= 8;
+    const int QD = a.n_head * HD;
+    int my_pid = 0;
+    auto page_of = [&](int i) {
+        if ((i & 63) == 0) my_pid = i + lane < n_pages ? a.table[(size_t)slot * a.max_pages + page_first + i + lane] : 0;
+        return __builtin_amdgcn_readlane(my_pid, i & 63);
+    };
+    h8 kreg[2 * KS], vreg[DT];
+    // (a page's block as one scalar address per four requests, which share the lane's offset)
+    auto load_page = [&](const __half * pool, int pid, auto & reg) {
+        uint64_t at = (uint64_t)(pool + (size_t)pid * a.page_stride + (size_t)h * a.head_stride);
+#pragma unroll
+        for (int j = 0; j < HD / 16; ++j) {
+            if (j > 0 && j % 4 == 0) { at += 4096; asm volatile("" : "+s"(at)); }
+            reg[j] = *(const h8 *)((const char *)at + lane * 16 + j % 4 * 1024);
+        }
+    };
+    auto load_k = [&](int pid) { load_page(a.k_pool, pid, kreg); };
+    auto load_v = [&](int pid) { load_page(a.v_pool, pid, vreg); };
+    int pid = page_of(0);
+    load_k(pid);
+    h8 q[KS];
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+        q[j] = load_h8((lo_col ? a.q_lo : a.q) + (size_t)t * QD + (size_t)(h * a.G + min(cc, a.G - 1)) * HD + 32 * j + 8 * g);
+    }
+    f4 o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d) o[d] = (f4){0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.0f;
+    if (shared) {
+        const int4 tm = a.tok_merge[t];
+        const float * part = a.partial + ((size_t)(tm.x + h * tm.y) * 16 + tm.z * a.G + min(cc, a.G - 1)) * PS;
+#pragma unroll
+        for (int u = 0; u < TAIL_SPLITS; ++u) m_run = fmaxf(m_run, part[(size_t)min(u, tm.y - 1) * 16 * PS]);
+#pragma unroll 1
+        for (int u = 0; u < tm.y; ++u, part += 16 * PS) {
+            const float2 ml = *(const float2 *)part;
+            const float w = ml.x == -INFINITY ? 0.0f : exp2f(ml.x - m_run);
+            l_run = fmaf(g == 0 ? w : 0.0f, ml.y, l_run);
+            const float wo = lo_col ? 0.0f : w;
+            const float2 * src = (const float2 *)(part + 2 + 4 * g);
+            float2 x[2 * DT];
+#pragma unroll
+            for (int d = 0; d < 2 * DT; ++d) x[d] = src[d / 2 * 8 + d % 2];
+            asm volatile("" : : : "memory");            // (all on their way before the first is waited for)
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                o[d][0] = fmaf(wo, x[2 * d].x, o[d][0]); o[d][1] = fmaf(wo, x[2 * d].y, o[d][1]);
+                o[d][2] = fmaf(wo, x[2 * d + 1].x, o[d][2]); o[d][3] = fmaf(wo, x[2 * d + 1].y, o[d][3]);
+            }
+        }
+    }
+    load_v(pid);
+#pragma unroll 1
+    for (int i = 0; i < n_pages; ++i) {
+        f4 s0 = (f4){0.f, 0.f, 0.f, 0.f}, s1 = (f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[2 * j], q[j], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[2 * j + 1], q[j], s1, 0, 0, 0);
+        }
+        if (i + 1 < n_pages) {
+            pid = page_of(i + 1);
+            load_k(pid);
+        }
+        // the hi and lo products of a query sit 8 columns apart: both lanes take the sum
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s0[e] += __shfl_xor(s0[e], 8, 64);
+            s1[e] += __shfl_xor(s1[e], 8, 64);
+        }
+        if (i + 1 == n_pages) {                   // positions past the row's own (the columns without a head are never stored)
+            const int last = pos - (page_first + i) * PAGE;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s0[e] = 4 * g + e <= last ? s0[e] : -INFINITY;
+                s1[e] = 16 + 4 * g + e <= last ? s1[e] : -INFINITY;
+            }
+        }
+        if (i == 0) {                             // and before the slot's first
+            const int first = kv_begin - page_first * PAGE;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s0[e] = 4 * g + e >= first ? s0[e] : -INFINITY;
+                s1[e] = 16 + 4 * g + e >= first ? s1[e] : -INFINITY;
+            }
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fmaxf(s0[e], s1[e]));
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = exp2f(m_run - m_use);       // m_run = -inf -> 0
+        m_run = m_new;
+        float psum = 0.0f;
+        h8 pt;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float e0 = exp2f(s0[e] - m_use), e1 = exp2f(s1[e] - m_use);
+            psum += e0 + e1;
+            const _Float16 h0 = (_Float16)e0, h1 = (_Float16)e1;
+            // the column of the lo query half multiplies the lo half of the same probabilities
+            pt[e] = lo_col ? (_Float16)(e0 - (float)h0) : h0;
+            pt[4 + e] = lo_col ? (_Float16)(e1 - (float)h1) : h1;
+        }
+        if (__any(alpha != 1.0f)) {
+            l_run *= alpha;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[d][e] *= alpha;
+        }
+        l_run += psum;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vreg[d], pt, o[d], 0, 0, 0);
+        if (i + 1 < n_pages) load_v(pid);
+    }
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    // the outputs against the lo halves of the probabilities join those against the hi halves
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[d][e] += __shfl_xor(o[d][e], 8, 64);
+    int t_out = t;               // (the places of the outputs are computed here, not kept in registers over the loop)
+    asm volatile("" : "+s"(t_out));
+    store_columns<HD>(a.out, o, l_run > 0.0f ? 1.0f / l_run : 0.0f, col_ok && !lo_col, t_out, h * a.G + cc, g, QD);
+}
+
+void attention_tail(hipStream_t s, const __half * q, const __half * q_lo, int n_rows, const AttnShape & sh, const PackBuffers & pk,
+                    const int32_t * table, int max_pages, const __half * k_pool, const __half * v_pool, const float * partial,
+                    const Act & out) {
+    if (n_rows <= 0) return;
+    if (!attention_decode_can(sh, 0)) throw std::runtime_error("attention_tail: unsupported shape or cache type");
+    check_act_out(out, sh.n_head * sh.head_dim, "attention_tail", n_rows);
+    if (!out.x) throw std::runtime_error("attention_tail: needs the plain activation planes");
+    if (sh.page_stride == 0 || sh.head_stride == 0) throw std::runtime_error("attention_tail: the pool's strides are missing");
+    if (!pk.dec_desc || !pk.tok_merge) throw std::runtime_error("attention_tail: the step's rows were not described");
+    TailArgs a {};
+    a.q = q; a.q_lo = q_lo; a.k_pool = k_pool; a.v_pool = v_pool; a.table = table; a.desc = pk.dec_desc; a.tok_merge = pk.tok_merge;
+    a.partial = partial; a.out = out; a.max_pages = max_pages; a.n_rows = n_rows;
+    a.n_head = sh.n_head; a.n_kv = sh.n_head_kv; a.G = sh.n_head / sh.n_head_kv;
+    a.page_stride = sh.page_stride; a.head_stride = sh.head_stride;
+    const dim3 grid((unsigned)((n_rows + 3) / 4 * sh.n_head_kv));
+    if (sh.head_dim == 128) hipLaunchKernelGGL(k_attention_tail<128>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_attention_tail<64>, grid, dim3(256), 0, s, a);
+    check_launch("attention_tail");
 }
 
 size_t attention_partial_floats(int n_items, int head_dim) {

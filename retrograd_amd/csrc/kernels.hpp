@@ -319,7 +319,7 @@ struct RowDesc {           // one per step row, written by the host
     int32_t sample;
     int32_t kv_begin;      // first resident position of the slot
     int32_t route;         // adapter route (0 = none)
-    int32_t pad;
+    int32_t shared;        // 1: the pages before kv_begin are attended beside other rows' (plan_shared_pages)
 };
 struct TableUpdate { int32_t slot; int32_t index; int32_t page; int32_t pad; };
 
@@ -380,6 +380,11 @@ int wide_tile_tokens(int G);
 // The step's work over its long rows; item numbers start at item0, `direct`: tiles that are not split leave their rows
 // themselves. Returns the number behind the last item.
 int plan_wide_attention(const RowDesc * rows, int n_rows, int G, int n_kv_heads, int wide_row, bool direct, int item0, std::vector<WideWork> & work);
+// The pages at the start of consecutive one-token rows that are the same pages (forked sequences), once per tile of rows instead
+// of once per row: the tiles' work as above, and kv_begin behind those pages in the rows they serve, whose own pages attention_tail
+// attends. (The rows beside it then show in the last bits of a row's result; the steps the launches are worth have 128 rows and more
+// over 8 kv heads.) pages: the page ids of every row's slot. Nothing (0) where reading them per row is as fast.
+int plan_shared_pages(RowDesc * rows, int n_rows, const int32_t * const * pages, int G, int n_kv_heads, std::vector<WideWork> & work);
 // Host mirror of the tile/item count (same formula as the kernel).
 void count_attention_work(const RowDesc * rows, int n_rows, int qt, int n_kv_heads, int wide_row,
                           int * n_tiles, int * n_items, int * split_pages);
@@ -450,6 +455,11 @@ bool attention_decode_can(const AttnShape & sh, int max_positions);
 void attention_decode(hipStream_t s, const float * qkv, const Slices & from, int n_rows, const AttnShape & sh,
                       const PackBuffers & pk, const int32_t * table, int max_pages, __half * k_pool, __half * v_pool,
                       const float * q_norm, const float * k_norm, const Act & out, unsigned long long * stamps = nullptr);
+// The rest of a decode step whose shared pages attention_wide has attended (plan_shared_pages; shapes as attention_decode_can): the
+// rows' own pages and the merge, after rope_store.
+void attention_tail(hipStream_t s, const __half * q, const __half * q_lo, int n_rows, const AttnShape & sh, const PackBuffers & pk,
+                    const int32_t * table, int max_pages, const __half * k_pool, const __half * v_pool, const float * partial,
+                    const Act & out);
 void attention_combine(hipStream_t s, const float * partial, int T, const AttnShape & sh,
                        const PackBuffers & pk, const Act & out);
 // Paged attention of the step's long rows (work on the device, n_work entries); tiles that are split leave partial
