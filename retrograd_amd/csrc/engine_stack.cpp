@@ -648,6 +648,19 @@ void Engine::plan_stack(const std::vector<RowView> & rows, const std::vector<std
         for (size_t r = 0; r < rows.size(); ++r)
             for (int64_t c = 0; c < (int64_t)rows[r].n * H; c += plan.cols) plan_blocks_.push_back({(int32_t)r, (int32_t)c});
         plan.n = plan_blocks_.size() - plan.first;
+        if (plan.n > 1) {           // longest first: what starts last is short
+            const int window = pair ? sp.attention.window : sp.latent.window, chunk = pair ? sp.attention.chunk : 0;
+            auto pages = [&](const rk::AttnBlock & b) {
+                const RowView & r = rows[(size_t)b.row];
+                const int lo = r.pos0 + b.col0 / H, hi = r.pos0 + std::min(b.col0 + cols - 1, (int)r.n * H - 1) / H;
+                const int reach = chunk > 0 ? lo - lo % chunk : window > 0 ? lo - window + 1 : 0;
+                return hi / rk::PAGE - std::max(slots_[(size_t)r.slot].begin, reach) / rk::PAGE + 1;
+            };
+            std::vector<std::pair<int, rk::AttnBlock>> by_length;
+            for (size_t i = plan.first; i < plan_blocks_.size(); ++i) by_length.push_back({pages(plan_blocks_[i]), plan_blocks_[i]});
+            std::stable_sort(by_length.begin(), by_length.end(), [](const auto & a, const auto & b) { return a.first > b.first; });
+            for (size_t i = 0; i < by_length.size(); ++i) plan_blocks_[plan.first + i] = by_length[i].second;
+        }
         block_plans_.push_back(plan);
     }
     if (!is_hybrid()) return;
