@@ -636,6 +636,10 @@ template <int KA, int KB> Slices run(hipStream_t s, int arith, DenseArgs & A, fl
             return out;
         }
     }
+    // A matrix per head: eight row tiles by a workgroup's four waves, which read the 64 tokens' operands together. (One row tile
+    // by eight waves along K read them once per row tile: 16 heads of 512 -> 128, 3321 tokens, 70 us, so 28; 128 -> 512 40, so
+    // 35.) Fewer than a workgroup per CU have more from the waves along K.
+    if (w.batch > 1 && T > 64 && (int64_t)((w.tiles + 7) / 8) * ((T + 63) / 64) * w.batch >= 256) { launch<uint16_t, KA, KB, 2, 4, 1, 4>(s, A); return out; }
     const bool deep = w.kf >= 16;
     if (deep && sliceable) slice_k(512 / std::max(T <= 16 ? w.tiles : (w.tiles + 1) / 2, 1), 64);
     if (!deep) {                        // one wave has too little of K to share it
