@@ -625,7 +625,51 @@ template <bool VEC> void launch_chunks(hipStream_t s, const MambaJob & j, int T)
     check_launch("mamba_chunk_out");
 }
 
-// act[t] = norm over each of the equal parts of (y * silu(z)), times the weight: one workgroup per token and part.
+// act[t] = norm over each of the equal parts of (y * silu(z)), times the weight, for parts of up to 1024 columns, a multiple of
+// eight: a wave per token and part, which stays in registers. (A workgroup of four waves had two columns per lane to wait for:
+// 3321 tokens of eight parts of 512 52 us, a wave
+// each 44, with four tokens per workgroup, whose activations are neighbours, 39; a copy of the bytes would take 28.)
+template <int ARITH>
+__global__ __launch_bounds__(256) void k_mamba_gate_norm_wave(MambaJob j, int T) {
+    constexpr int GROUPS = 2;             // of eight columns per lane
+    const int inner = j.sh.inner(), len = inner / j.sh.norm_groups;
+    // (the activations of four tokens lie side by side)
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), k0 = blockIdx.y * len, lane = threadIdx.x & 63;
+    if (t >= T) return;
+    const float * y = j.y + (size_t)t * inner + k0, * z = j.proj + (size_t)t * j.ld + k0, * weight = j.norm_w + k0;
+    f4 a[GROUPS][2], b[GROUPS][2], wt[GROUPS][2];
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = min(8 * (lane + 64 * g), len - 8) + 4 * u;
+            a[g][u] = *(const f4 *)(y + k);
+            b[g][u] = *(const f4 *)(z + k);
+            wt[g][u] = *(const f4 *)(weight + k);
+        }
+    float q = 0.0f;
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                a[g][u][e] *= silu_f(b[g][u][e]);
+                if (8 * (lane + 64 * g) < len) q += a[g][u][e] * a[g][u][e];
+            }
+    const float inv = 1.0f / sqrtf(wave_sum(q) / (float)len + j.eps);
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+        const int k = 8 * (lane + 64 * g);
+        if (k >= len) continue;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = a[g][e / 4][e % 4] * inv * wt[g][e / 4][e % 4];
+        store_frag8<ARITH>(j.out, j.out_kf, t, k0 + k, v);
+    }
+}
+
+// ... and of any other: one workgroup per token and part.
 template <int ARITH>
 __global__ __launch_bounds__(256) void k_mamba_gate_norm(MambaJob j) {
     extern __shared__ float row[];
@@ -696,6 +740,14 @@ void mamba_mix(hipStream_t s, int arith, const MambaJob & j, int T) {
         // every row starts at a multiple of four floats
         if (sh.vdim % 4 == 0 && sh.state % 4 == 0) launch_chunks<true>(s, c, T);
         else launch_chunks<false>(s, c, T);
+    }
+    const int len = sh.inner() / sh.norm_groups;
+    if (len % 8 == 0 && len <= 1024 && sh.inner() % 4 == 0 && j.ld % 4 == 0) {
+        const dim3 grid((unsigned)((T + 3) / 4), (unsigned)sh.norm_groups);
+        if (arith == ARITH_16) hipLaunchKernelGGL(k_mamba_gate_norm_wave<ARITH_16>, grid, dim3(256), 0, s, j, T);
+        else hipLaunchKernelGGL(k_mamba_gate_norm_wave<ARITH_32>, grid, dim3(256), 0, s, j, T);
+        check_launch("mamba_gate_norm");
+        return;
     }
     const dim3 gn((unsigned)T, (unsigned)sh.norm_groups);
     const size_t nl = (size_t)(sh.inner() / sh.norm_groups) * 4;

@@ -9,6 +9,8 @@ namespace {
 
 constexpr int kConvTokens = 16;       // tokens of a run one workgroup convolves
 
+// What bounds it is the bytes, in and out (33 us at a copy's rate for 3321 tokens of 6144 channels): a thread that asked for a
+// token's input when it had stored the one before took 67 us, with all sixteen on their way 36.
 template <int TAPS>
 __global__ __launch_bounds__(256) void k_short_conv(ShortConv j) {
     const int C = j.channels, c = blockIdx.y * 256 + threadIdx.x, K = TAPS > 0 ? TAPS : j.taps;
@@ -26,22 +28,24 @@ __global__ __launch_bounds__(256) void k_short_conv(ShortConv j) {
     const float * w = j.w + (size_t)c * K;
     const float bias = j.b ? j.b[c] : 0.0f;
     const int last = min(first + kConvTokens, run.n);
-    if constexpr (TAPS > 0) {                   // the window and the taps in registers
-        float win[TAPS], tap[TAPS];
+    if constexpr (TAPS > 0) {                   // the taps and all inputs in registers, requested together
+        float tap[TAPS], x[TAPS - 1 + kConvTokens];
 #pragma unroll
-        for (int k = 0; k < TAPS; ++k) {
-            tap[k] = w[k];
-            win[k] = k > 0 ? input(first - TAPS + k) : 0.0f;
+        for (int k = 0; k < TAPS; ++k) tap[k] = w[k];
+#pragma unroll
+        for (int k = 0; k < TAPS - 1; ++k) x[k] = input(first - (TAPS - 1) + k);
+#pragma unroll
+        for (int i = 0; i < kConvTokens; ++i) {          // (by fours: a short run asks for few)
+            x[TAPS - 1 + i] = 0.0f;
+            if (first + i / 4 * 4 < last) x[TAPS - 1 + i] = j.in[(size_t)j.runs.tok[run.start + min(first + i, last - 1)] * j.ld + c];
         }
-        for (int i = first; i < last; ++i) {
-            const int t = j.runs.tok[run.start + i];
+#pragma unroll
+        for (int i = 0; i < kConvTokens; ++i) {
+            if (first + i >= last) continue;
             float v = 0.0f;
 #pragma unroll
-            for (int k = 0; k + 1 < TAPS; ++k) win[k] = win[k + 1];
-            win[TAPS - 1] = j.in[(size_t)t * j.ld + c];
-#pragma unroll
-            for (int k = 0; k < TAPS; ++k) v += tap[k] * win[k];
-            j.out[(size_t)t * C + c] = silu_f(v + bias);
+            for (int k = 0; k < TAPS; ++k) v += tap[k] * x[i + k];
+            j.out[(size_t)j.runs.tok[run.start + first + i] * C + c] = silu_f(v + bias);
         }
     } else {
         for (int i = first; i < last; ++i) {
