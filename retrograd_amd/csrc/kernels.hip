@@ -1057,7 +1057,7 @@ __global__ __launch_bounds__(NW * 64) void k_rmsnorm_act8(float * x, const float
                                                           Slices add) {
     constexpr int STEP = NW * 64 * 8;
     __shared__ float red[NW];
-    const int o = blockIdx.x;
+    const int o = row_of_block(blockIdx.x, gridDim.x);
     const int row = rows ? rows[o] : o;
     float * xr = x + (size_t)row * E;
     float ss = 0.0f;
@@ -1751,7 +1751,7 @@ struct RopeArgs {
 // One wave per head: lanes own element pairs.
 __global__ __launch_bounds__(256) void k_rope_store(RopeArgs a) {
     __shared__ float stash[4][128];          // Q8_0 cache: a head's row in element order, per wave
-    const int t = blockIdx.x;
+    const int t = row_of_block(blockIdx.x, gridDim.x);
     const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int heads_total = a.n_head + 2 * a.n_kv;
@@ -2832,7 +2832,7 @@ struct CombineArgs {
 // the splits are read one per lane, the outputs two dimensions per lane.
 __global__ __launch_bounds__(256) void k_attention_combine(CombineArgs a) {
     __shared__ float blk_amax[4], blk_first[4];
-    const int t = blockIdx.x;
+    const int t = row_of_block(blockIdx.x, gridDim.x);
     const int wave = threadIdx.x >> 6;
     const int head = blockIdx.y * 4 + wave;
     const int lane = threadIdx.x & 63;

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(1024) void k_norm_act(float * __restrict__ x, const
                                                    const float * __restrict__ plus, void * __restrict__ act_rows) {
     extern __shared__ __attribute__((aligned(16))) float row[];
     __shared__ float scratch[16];
-    const int t = rows ? rows[blockIdx.x] : (int)blockIdx.x, n_thr = blockDim.x;
+    const int o = row_of_block(blockIdx.x, gridDim.x), t = rows ? rows[o] : o, n_thr = blockDim.x;
     float * xr = x + (size_t)t * E;
     float sum = 0.0f;
     if constexpr (VEC) {
@@ -67,8 +67,8 @@ __global__ __launch_bounds__(1024) void k_norm_act(float * __restrict__ x, const
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = k + i < E ? (row[k + i] - mean) * inv * w[k + i] : 0.0f;
-        store_frag8<ARITH>(act, kf, blockIdx.x, k, v);
-        if (act_rows) store_act8_at<ARITH>(act_rows, (size_t)blockIdx.x * kf * 32 + k, v);
+        store_frag8<ARITH>(act, kf, o, k, v);
+        if (act_rows) store_act8_at<ARITH>(act_rows, (size_t)o * kf * 32 + k, v);
     }
 }
 
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(1024) void k_streams_norm_act(Streams x, const floa
     extern __shared__ __attribute__((aligned(16))) float row[];
     __shared__ float scratch[16];
     using Columns = StreamColumns<N, W>;
-    const int t = rows ? rows[blockIdx.x] : (int)blockIdx.x, n_thr = blockDim.x;
+    const int o = row_of_block(blockIdx.x, gridDim.x), t = rows ? rows[o] : o, n_thr = blockDim.x;
     float sum = 0.0f;
     for (int k = W * (int)threadIdx.x; k < E; k += W * n_thr) {
         const size_t at = (size_t)t * E + k;
@@ -140,8 +140,8 @@ __global__ __launch_bounds__(1024) void k_streams_norm_act(Streams x, const floa
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = k + i < E ? row[k + i] * inv * w[k + i] : 0.0f;
-        store_frag8<ARITH>(act, kf, blockIdx.x, k, v);
-        if (act_rows) store_act8_at<ARITH>(act_rows, (size_t)blockIdx.x * kf * 32 + k, v);
+        store_frag8<ARITH>(act, kf, o, k, v);
+        if (act_rows) store_act8_at<ARITH>(act_rows, (size_t)o * kf * 32 + k, v);
     }
 }
 
@@ -220,8 +220,9 @@ __global__ __launch_bounds__(1024) void k_sublayer_norm(SublayerNorm j) {
     const int E = j.E, n_thr = blockDim.x, wave = threadIdx.x >> 6, waves = n_thr >> 6;
     SeqRun run = {};
     if constexpr (OUT == NORM_CONVOLVED) run = j.runs.runs[blockIdx.x];
-    const int t = OUT == NORM_CONVOLVED ? j.runs.tok[run.start] : j.rows ? j.rows[blockIdx.x] : (int)blockIdx.x;
-    const int at = OUT == NORM_CONVOLVED ? t : (int)blockIdx.x;              // row of the activations
+    const int o = row_of_block(blockIdx.x, gridDim.x);
+    const int t = OUT == NORM_CONVOLVED ? j.runs.tok[run.start] : j.rows ? j.rows[o] : o;
+    const int at = OUT == NORM_CONVOLVED ? t : o;              // row of the activations
     const int past = OUT == NORM_CONVOLVED ? j.n_taps - 1 : 0, plane = (run.flags >> 1) & 1;
     const bool fresh = run.flags & 1;
     const float * old_in = nullptr;

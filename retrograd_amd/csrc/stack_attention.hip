@@ -25,7 +25,7 @@ __global__ __launch_bounds__(256) void k_latent_norms(LatentNorms a) {
     using EL = typename std::conditional<ARITH == ARITH_16, __half, float>::type;
     __shared__ float scratch[16];
     constexpr int KEEP = 2;                    // groups of eight per thread that stay in registers
-    const int t = blockIdx.x;
+    const int t = row_of_block(blockIdx.x, gridDim.x);
     const bool kv = blockIdx.y == 1;
     const int n = kv ? a.kv_rank : a.q_rank;
     const float * src = a.proj + (size_t)t * a.ld + (kv ? a.kv_col : 0);
@@ -96,7 +96,7 @@ template <int ARITH>
 __global__ __launch_bounds__(256) void k_head_rows(HeadRows a) {
     using EL = typename std::conditional<ARITH == ARITH_16, __half, float>::type;
     __shared__ float scratch[16];
-    const int t = blockIdx.x;
+    const int t = row_of_block(blockIdx.x, gridDim.x);
     const float * row = a.proj + (size_t)t * a.ld;
     auto squares = [&](const float * x, int n) {       // rows start at multiples of four columns
         float q = 0.0f;
