@@ -461,7 +461,7 @@ class _ResultBuffers:
         self._closed = False
 
     def take(self, shape) -> np.ndarray:
-        n = int(np.prod(shape)) * 4
+        n = shape[0] * shape[1] * 4
         if n < self.MIN_BYTES or n > self.LIMIT_BYTES or self._closed:
             return np.empty(shape, np.float32)
         at, size = self._fitting(n)
