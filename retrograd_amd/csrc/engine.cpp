@@ -1589,7 +1589,7 @@ void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_row
                 const int cols[3] = {0, QD, QD + KD}, widths[3] = {QD, KD, KD};
                 const rk::LoraEntry * tables[3] = {lora_entries(l, 0), lora_entries(l, 1), lora_entries(l, 2)};
                 rk::lora_apply_targets(stream_, 3, tables, widths, cols, rows_d, pk_.row, act_e, T, dst, QD + 2 * KD,
-                                       lora_mid_.as<float>());
+                                       lora_mid_.as<float>(), lora_max_rank_);
             }
             prof_end(PC_QKV, pt_);
         }
@@ -1628,7 +1628,7 @@ void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_row
             if (routed) {
                 float * dst = pending.n > 0 ? const_cast<float *>(pending.data) : x;
                 rk::lora_apply(stream_, lora_entries(l, 3), d_stage_.as<rk::RowDesc>(), pk_.row, act_q, T, E, dst, E, 0,
-                               lora_mid_.as<float>());
+                               lora_mid_.as<float>(), lora_max_rank_);
             }
             prof_end(PC_OPROJ, pt_);
         } else {
@@ -1669,7 +1669,7 @@ void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_row
         if (routed) {
             float * dst = pending.n > 0 ? const_cast<float *>(pending.data) : x;
             rk::lora_apply(stream_, lora_entries(l, 3), d_stage_.as<rk::RowDesc>(), pk_.row, act_q, T, E, dst, E, 0,
-                           lora_mid_.as<float>());
+                           lora_mid_.as<float>(), lora_max_rank_);
         }
         prof_end(PC_OPROJ, pt_);
         }
@@ -1734,7 +1734,7 @@ void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_row
                 const int cols[2] = {0, group}, widths[2] = {F, F};
                 const rk::LoraEntry * tables[2] = {lora_entries(l, 4), lora_entries(l, 5)};
                 rk::lora_apply_targets(stream_, 2, tables, widths, cols, d_stage_.as<rk::RowDesc>(), pk_.row, act_e, T, gu,
-                                       2 * F, lora_mid_.as<float>(), L.gate_up_interleaved ? group : 0);
+                                       2 * F, lora_mid_.as<float>(), lora_max_rank_, L.gate_up_interleaved ? group : 0);
             }
             prof_end(PC_GATEUP, pt_);
             pt_ = prof_begin(PC_SWIGLU);
@@ -1746,7 +1746,7 @@ void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_row
         if (ffn_lora) {
             float * dst = pending.n > 0 ? const_cast<float *>(pending.data) : x;
             rk::lora_apply(stream_, lora_entries(l, 6), d_stage_.as<rk::RowDesc>(), pk_.row, act_f, T, E, dst, E, 0,
-                           lora_mid_.as<float>());
+                           lora_mid_.as<float>(), lora_max_rank_);
         }
         prof_end(PC_DOWN, pt_);
     }
@@ -2050,11 +2050,13 @@ int Engine::adapter_unload(int32_t id) {
 void Engine::rebuild_lora_table() {
     lora_routes_ = (int)row_adapters_.size();
     lora_has_ffn_ = false;
+    lora_max_rank_ = 0;
     if (lora_routes_ == 0) return;
     std::vector<rk::LoraEntry> table((size_t)hp_.n_layer * kLoraTargets * (size_t)lora_routes_);
     int route = 0;
     for (const auto & kv : row_adapters_) {
         const RowAdapterData & d = kv.second;
+        lora_max_rank_ = std::max(lora_max_rank_, (int)d.rank);
         for (int l = 0; l < hp_.n_layer; ++l)
             for (int tg = 0; tg < kLoraTargets; ++tg) {
                 rk::LoraEntry & e = table[((size_t)l * kLoraTargets + tg) * (size_t)lora_routes_ + (size_t)route];

@@ -493,7 +493,7 @@ private:
     int32_t next_adapter_id_ = 1;
     DevBuf lora_table_;       // LoraEntry [layer][target][route - 1]
     DevBuf lora_mid_;         // [n_batch][LORA_MAX_RANK] f32
-    int lora_routes_ = 0;
+    int lora_routes_ = 0, lora_max_rank_ = 0;
     bool ggml_activations_ = false;   // RETRO_ACTIVATIONS=ggml at construction
     bool moe_scaled_ = false;         // RETRO_MOE_SCALED=1: decode-sized steps multiply MXFP4 experts on the block-scaled matrix
                                       // instruction (measured slower than the f16 tile kernels end to end, so it is off by default)

@@ -244,15 +244,15 @@ constexpr int LORA_MAX_RANK = 64;
 // For every token whose row routes to an adapter (rows[tok_row[t]].route > 0,
 // entry table[route - 1], skipped when the entry has no pair for this target):
 //   y[t][col0 + n] += scale * sum_r B[n][r] * (sum_k A[r][k] * x[t][k]).
-// mid is scratch of T * LORA_MAX_RANK floats.
+// mid is scratch of T * LORA_MAX_RANK floats, max_rank the largest rank in the table.
 // The same for up to three targets that read the same activations (tables[i], widths[i], cols[i]), in one
 // pair of launches; mid is scratch of n_targets * T * LORA_MAX_RANK floats. group > 0: output n of a target
 // lands in column cols[i] + (n / group) * 2 group + n % group (gate and up outputs interleaved by `group`).
 void lora_apply_targets(hipStream_t s, int n_targets, const LoraEntry * const * tables, const int * widths, const int * cols,
                         const RowDesc * rows, const int32_t * tok_row, const Act & x, int T, float * y, int ldy, float * mid,
-                        int group = 0);
+                        int max_rank, int group = 0);
 void lora_apply(hipStream_t s, const LoraEntry * table, const RowDesc * rows, const int32_t * tok_row,
-                const Act & x, int T, int N, float * y, int ldy, int col0, float * mid);
+                const Act & x, int T, int N, float * y, int ldy, int col0, float * mid, int max_rank);
 // out[r][k] = decode(raw row r)[k] as f32: any tensor to f32, row by row.
 void decode_rows(hipStream_t s, int type, const uint8_t * raw, int K, int n_rows, float * out);
 

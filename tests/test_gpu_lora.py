@@ -310,3 +310,38 @@ def test_adapter_errors_and_unload(files):
     assert eng.adapter_load(a2) == 2, "ids are never reused"
     assert eng.adapter_rows_info().n_adapters == 1
     eng.close()
+
+
+def test_adapters_of_all_ranks_in_small_and_large_steps(tmp_path):
+    """Ranks that are no multiple of four, of sixteen, or the largest, over rows of 4352 columns: rows decoded alone (factors
+    asked for ahead) and 45 at once (more workgroups than that form takes) give the same logits. Operands carry 22 bits and sums
+    are f32, about 1e-6 of the logits: 1e-5 is asked of nine rows in ten; a new key or value may sit on the other side of a rounding
+    boundary of the f16 cache (2^-11 of a value, in one dimension of a head whose whole weight lies on that token)."""
+    shape = synth.scaled(synth.QWEN25_7B_Q8, n_layer=1, n_embd=4352, n_head=8, n_head_kv=2, head_dim=64, n_ff=512, n_vocab=512, name="lora-ranks")
+    model = tmp_path / "m.gguf"
+    synth.write_model(model, shape, seed=9, device="cpu", std=0.02)
+    with E.Engine(model, E.EngineConfig(n_ctx=2048, n_seq_max=45, n_batch=128, n_ubatch=128)) as eng:
+        ids = [E.RETRO_STEP_ADAPTER_BASE]
+        for rank in (5, 20, 64):
+            path = tmp_path / ("r%d.gguf" % rank)
+            synth.write_lora_adapter(path, shape, rank=rank, alpha=2.0 * rank, seed=rank, std_a=0.05, std_b=0.05)
+            ids.append(eng.adapter_load(path, 1.0))
+        rng = np.random.default_rng(2)
+        out = E.StepOutput()
+        lens = [3 + i % 7 for i in range(45)]
+        row = lambda i, tokens, pos: E.StepRow(i, i, tokens, pos, sample=True, sampling=greedy(), adapter=E.RowAdapter(ids[i % 4]))
+        for i in range(45):
+            eng.step([row(i, rng.integers(0, shape.n_vocab, lens[i]), 0)], out)
+        new = [[int(t)] for t in rng.integers(0, shape.n_vocab, 45)]
+        alone = []
+        for i in range(45):
+            eng.step([row(i, new[i], lens[i])], out)
+            alone.append(eng.debug_logits()[0].copy())
+            eng.seq_rm(i, lens[i], lens[i] + 1)
+        eng.step([row(i, new[i], lens[i]) for i in range(45)], out)
+        got, alone = eng.debug_logits(), np.stack(alone)
+        worst = np.linalg.norm(got - alone, axis=1) / np.linalg.norm(alone, axis=1)
+        print("nine of ten %.2e, worst row %.2e" % (np.quantile(worst, 0.9), worst.max()), flush=True)
+        assert np.isfinite(got).all() and np.quantile(worst, 0.9) <= 1e-5 and worst.max() <= 2.0 ** -11 / np.sqrt(64 / 3)
+        for r in range(1, 4):      # each adapter does something
+            assert np.abs(alone[r] - alone[r - 1]).max() > 1e-2
