@@ -1596,7 +1596,7 @@ void Engine::forward(int T, int n_out, const AttnPlan & plan, bool one_token_row
         size_t pt_;
         if (fused_decode) {
             unsigned long long * stamps = nullptr;
-            if (attn_timeline_ && l == h.n_layer / 2) {
+            if (attn_timeline_ && plan.n_wide == 0 && l == h.n_layer / 2) {
                 attn_stamped_wgs_ = (size_t)T * (size_t)h.n_head_kv;
                 attn_stamps_.ensure(attn_stamped_wgs_ * 6 * sizeof(unsigned long long));
                 stamps = attn_stamps_.as<unsigned long long>();
