@@ -185,14 +185,20 @@ __device__ __forceinline__ void store_rows(const DenseJob & j, int t, int b, int
 }
 
 // An expert's rows of the pair in slot t.
-__device__ __forceinline__ void store_expert(const DenseArgs & A, int t, int n, f4 v) {
+// (The slot's place and weight are looked up once per slot, ahead of the product: looked up at every store they made each store
+// wait for the one before: 31200 pairs of 768 -> 2048 columns 231 us, so 208.)
+struct ExpertRow { float * y; float w; };
+__device__ __forceinline__ ExpertRow expert_row(const DenseArgs & A, int t) {
     const DenseOut & o = A.j.a;
+    const int pair = A.groups.slot_pair[t], token = pair / A.groups.top, choice = pair - token * A.groups.top;
+    return {(float *)o.dst + (size_t)choice * o.stride + (size_t)token * o.ld, A.groups.weigh_input ? 1.0f : A.groups.weight[pair]};
+}
+__device__ __forceinline__ void store_expert(const DenseArgs & A, const ExpertRow & row, int n, f4 v) {
     const int cnt = A.j.w.n - n;
     if (cnt <= 0) return;
-    const int pair = A.groups.slot_pair[t], token = pair / A.groups.top, choice = pair - token * A.groups.top;
-    if (!A.groups.weigh_input) v *= A.groups.weight[pair];
-    float * y = (float *)o.dst + (size_t)choice * o.stride + (size_t)token * o.ld + n;
-    if (cnt >= 4 && (o.ld & 3) == 0) *(f4 *)y = v;
+    if (!A.groups.weigh_input) v *= row.w;
+    float * y = row.y + n;
+    if (cnt >= 4 && (A.j.a.ld & 3) == 0) *(f4 *)y = v;
     else
         for (int i = 0; i < 4 && i < cnt; ++i) y[i] = v[i];
 }
@@ -382,6 +388,11 @@ __global__ __launch_bounds__(64 * KW * RW) void k_dense(DenseArgs A) {
         }
         if (kw != 0) return;
     }
+    ExpertRow out_row[KA == OUT_EXPERT ? CT : 1];
+    if constexpr (KA == OUT_EXPERT) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) out_row[c] = expert_row(A, min(cols.first + c * 16 + (lane & 15), cols.end - 1));
+    }
     constexpr int ARITH = (int)sizeof(TA);
     if constexpr (DUAL) {
 #pragma unroll
@@ -408,7 +419,7 @@ __global__ __launch_bounds__(64 * KW * RW) void k_dense(DenseArgs A) {
             const int t = cols.first + c * 16 + (lane & 15);
             if (t >= cols.end) continue;
             if constexpr (KA == OUT_EXPERT) {
-                store_expert(A, t, tile * 16 + 4 * (lane >> 4), acc[r][c]);
+                store_expert(A, out_row[c], tile * 16 + 4 * (lane >> 4), acc[r][c]);
             } else if (DUAL && A.partial) {
                 store_slice(A, ks, t, tile * 16 + 4 * (lane >> 4), acc[r][c], false);
             } else {
@@ -450,10 +461,15 @@ __global__ __launch_bounds__(256, 2) void k_dense_lds(DenseArgs A, int n_tok_blo
     // that its concurrent workgroups share both operands in its L2
     const int n_groups = A.n_groups;
     int gb, tb, ks;
-    if constexpr (GROUPED) {           // the row blocks of a tile of slots on one XCD, which keeps the gathered rows in its L2
-        const int i = blockIdx.x >> 3;
+    if constexpr (GROUPED) {
+        // The row blocks of a tile of slots on one XCD, which keeps the gathered rows in its L2, and the tiles of an expert, which
+        // follow each other, on one as well, which then reads the expert's weights once (with the tiles dealt in turn every tile's
+        // XCD did: by the counters 0.9 GB for the 250 MB of 31200 pairs through 64 experts of 768 -> 2048 columns;
+        // the product into them, 2048 -> 2 x 768, 273 us, so 231).
+        const int i = blockIdx.x >> 3, nth = i / n_groups, per = (*A.groups.n_tiles + 7) / 8;
+        if (nth >= per) return;
         gb = i % n_groups;
-        tb = (i / n_groups) * 8 + (blockIdx.x & 7);
+        tb = (int)(blockIdx.x & 7) * per + nth;
         ks = 0;
     } else {
         const int b = A.ksplit > 1 ? blockIdx.x % A.grid_k : blockIdx.x;
@@ -468,6 +484,11 @@ __global__ __launch_bounds__(256, 2) void k_dense_lds(DenseArgs A, int n_tok_blo
     if (!columns_of<GROUPED>(A, tb, cols)) return;
     const int tile0 = gb * 2 * RT;
     const uint16_t * weights = j.w.w + (size_t)cols.b * j.w.tiles * j.w.kf * 512;
+    ExpertRow out_row[KA == OUT_EXPERT ? CT : 1];
+    if constexpr (KA == OUT_EXPERT) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) out_row[c] = expert_row(A, min(cols.first + (wt * CT + c) * 16 + (lane & 15), cols.end - 1));
+    }
     f4 acc[RT][CT];
     auto clear = [&]() {
 #pragma unroll
@@ -554,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void k_dense_lds(DenseArgs A, int n_tok_blo
                     if (biased) v += bias_of(j, 0, tile, lane >> 4);
                 }
                 if constexpr (KA == OUT_EXPERT) {
-                    store_expert(A, t, tile * 16 + 4 * (lane >> 4), v);
+                    store_expert(A, out_row[c], tile * 16 + 4 * (lane >> 4), v);
                 } else if (DUAL && A.partial) {
                     store_slice(A, ks, t, tile * 16 + 4 * (lane >> 4), v, !first);
                 } else {
@@ -688,8 +709,8 @@ template <int KA> void run_groups(hipStream_t s, int arith, DenseArgs & A) {
         case 16: deep ? launch_groups<uint16_t, KA, R1, 1, 8, 1>(s, A) : launch_groups<uint16_t, KA, R1, 1, 1, 4>(s, A); break;
         case 32: deep ? launch_groups<uint16_t, KA, 2, 2, 8, 1>(s, A) : launch_groups<uint16_t, KA, R1, 2, 1, 4>(s, A); break;
         case 64: launch_lds_groups<KA, 4, 2>(s, A); break;
-        default:
-            if (out_is_glu(KA) && (int64_t)A.groups.max_tiles * ((A.j.w.tiles + 15) / 16) >= 448) launch_lds_groups<KA, 8, 4>(s, A);
+        default:       // (rows of the experts' outputs 205 us with 128-row tiles, 177 with 256)
+            if ((int64_t)A.groups.max_tiles * ((A.j.w.tiles + 15) / 16) >= 448) launch_lds_groups<KA, 8, 4>(s, A);
             else launch_lds_groups<KA, 4, 4>(s, A);
             break;
     }
