@@ -546,6 +546,32 @@ __global__ __launch_bounds__(256, 2) void k_dense_lds(DenseArgs A, int n_tok_blo
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // nothing may land in LDS that another workgroup owns by then
     };
     auto store = [&](const float * scale, bool first) {
+        // What the residual's rows are scaled with, and the residual itself, are asked for together: a load behind a store waits
+        // for the store (3321 tokens, 12288 -> 2048 columns 191 us, so 185; 2048 -> 2048 at 3900 tokens 45, so 42).
+        constexpr int PR = DUAL ? RT : 1, PC = DUAL ? CT : 1;
+        float factor[PC];
+        f4 scales[PR], before[PR][PC];
+        const bool direct = DUAL && !A.partial && ((j.a.ld | j.a.col0) & 3) == 0;
+        auto column_at = [&](int r) { return (tile0 + wn * RT + r) * 16 + 4 * (lane >> 4); };
+        if constexpr (DUAL) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) factor[c] = token_factor(j, min(cols.first + (wt * CT + c) * 16 + (lane & 15), cols.end - 1));
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                scales[r] = f4{1, 1, 1, 1};
+                const int n = column_at(r);
+                if (scale) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) scales[r][i] = n + i < j.w.n ? scale[n + i] : 0.0f;
+                }
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const int t = cols.first + (wt * CT + c) * 16 + (lane & 15);
+                    before[r][c] = f4{0, 0, 0, 0};
+                    if (direct && t < cols.end && n + 4 <= j.n_a) before[r][c] = *(const f4 *)((const float *)j.a.dst + (size_t)t * j.a.ld + j.a.col0 + n);
+                }
+            }
+        }
         const bool biased = j.bias && ks == 0 && first;
         if (!DUAL && biased) {
 #pragma unroll
@@ -559,25 +585,21 @@ __global__ __launch_bounds__(256, 2) void k_dense_lds(DenseArgs A, int n_tok_blo
         for (int r = 0; r < RT; ++r) {
             const int tile = tile0 + wn * RT + r;
             if (tile >= j.w.tiles) break;
-            f4 f = {1, 1, 1, 1};
-            if (scale) {
-                const int n = tile * 16 + 4 * (lane >> 4);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) f[i] = n + i < j.w.n ? scale[n + i] : 0.0f;
-            }
 #pragma unroll
             for (int c = 0; c < CT; ++c) {
                 const int t = cols.first + (wt * CT + c) * 16 + (lane & 15);
                 if (t >= cols.end) continue;
                 f4 v = acc[r][c];
                 if constexpr (DUAL) {
-                    v *= f * token_factor(j, t);
+                    v *= scales[r] * factor[c];
                     if (biased) v += bias_of(j, 0, tile, lane >> 4);
                 }
                 if constexpr (KA == OUT_EXPERT) {
                     store_expert(A, out_row[c], tile * 16 + 4 * (lane >> 4), v);
                 } else if (DUAL && A.partial) {
                     store_slice(A, ks, t, tile * 16 + 4 * (lane >> 4), v, !first);
+                } else if (DUAL && direct && column_at(r) + 4 <= j.n_a) {
+                    *(f4 *)((float *)j.a.dst + (size_t)t * j.a.ld + j.a.col0 + column_at(r)) = v + before[r][c];
                 } else {
                     f4 next = acc[r ^ 1][c];
                     if constexpr (GROUPED) {
